@@ -106,6 +106,12 @@ struct sph_ctx {
     // sort: hash keys (pre-sort order), ping-pong keys/vals, sorted result
     uint32_t *key_h = nullptr, *key_t = nullptr, *key_s = nullptr;
     uint32_t *val_t = nullptr, *val_s = nullptr;
+    // canonical order: slots per cell and each slot's number in its cell (arr is
+    // val_t, the slots by cell key_t: the sort's buffers), and the scan's words
+    uint32_t *ccount = nullptr;
+    unsigned long long *scan_state = nullptr;
+    uint32_t ccount_cap = 0;
+    bool by_counts = false;   // the layout's grid phase sorts by counts (else by digits)
     uint32_t *hist = nullptr;
     uint32_t *partials = nullptr;
     uint32_t *cstart = nullptr;
@@ -186,6 +192,15 @@ struct sph_ctx {
         s.vx = vel[which][0]; s.vy = vel[which][1]; s.vz = vel[which][2];
         s.id = ids[idw];
         return s;
+    }
+
+    // the counts of the keys the next grid phase sorts (none when it sorts by digits)
+    sph::CellCount counts() const
+    {
+        sph::CellCount cc;
+        cc.count = by_counts ? ccount : nullptr;
+        cc.arr = val_t;
+        return cc;
     }
 
     bool ref_order() const { return (flags & SPH_FLAG_REFERENCE_ORDER) != 0; }
@@ -437,6 +452,28 @@ std::vector<uint32_t> scenes_by_slot(const sph_ctx *c)
     return order;
 }
 
+// Whether the grid phase sorts by the cells' counts (k_scan_chained, k_place,
+// k_gather) rather than by digits of the keys. The counts are read, scanned and
+// cleared cell by cell, about 6 us a million cells, the digit passes only write the
+// table (about 2.5 us), but cost two launches of three kernels and more per slot:
+// 20 us at 20,000 slots, 48 us at a million. Measured grid phases, counts against
+// digits: 20,000 slots in 27,000 cells 20.6 / 39.6 us, in 8.0 M cells 79.2 / 79.1;
+// 100,000 slots in 2.1 M cells 36 / 69 us, 8.0 M 71 / 77, 17 M 117 / 93; 1,000,000
+// slots in 8.0 M cells 89 / 109 us, in 27 M 207 / 151.
+bool sort_by_counts(uint32_t cells, uint32_t slots)
+{
+    return cells <= (8ull << 20) + 6ull * slots;
+}
+
+// Zeroes the cell counts (and the scan's words): no key is counted.
+sph_status clear_counts(sph_ctx *c)
+{
+    if (!c->by_counts) return SPH_OK;
+    SPH_HIP(hipMemsetAsync(c->ccount, 0, (size_t) c->ccount_cap * sizeof(uint32_t), c->stream));
+    SPH_HIP(hipMemsetAsync(c->scan_state, 0, (size_t) sph::scan_state_words(c->ccount_cap) * 8, c->stream));
+    return SPH_OK;
+}
+
 // Rebuilds the segment table from the scenes (host counts must be current) and
 // uploads it with the group map and the emitters.
 sph_status rebuild_layout(sph_ctx *c)
@@ -520,6 +557,24 @@ sph_status rebuild_layout(sph_ctx *c)
         SPH_TRY(dalloc(c, &c->cstart, want));
         c->cstart_cap = want;
     }
+    c->by_counts = !c->ref_order() && sort_by_counts(c->total_cells, c->nslots);
+    if (c->by_counts && c->total_cells + 1 > c->ccount_cap) {
+        dfree(c, c->ccount);
+        dfree(c, c->scan_state);
+        c->ccount = nullptr;
+        c->scan_state = nullptr;
+        c->ccount_cap = 0;
+        if (dalloc(c, &c->ccount, c->cstart_cap) == SPH_OK &&
+            dalloc(c, &c->scan_state, (size_t) sph::scan_state_words(c->cstart_cap)) == SPH_OK) {
+            c->ccount_cap = c->cstart_cap;
+        } else {   // no room for the counts: the digit passes need none
+            (void) hipGetLastError();
+            dfree(c, c->ccount);
+            c->ccount = nullptr;
+            c->by_counts = false;
+        }
+    }
+    SPH_TRY(clear_counts(c));
     if (c->ref_order()) {
         if (c->total_cells + 1 > c->ref_cells_cap) {
             for (uint32_t **a : {&c->ref.n_early, &c->ref.n_arrive, &c->ref.n_depart, &c->ref.nstay, &c->ref.partials}) {
@@ -630,8 +685,10 @@ bool find_range(const sph_ctx *c, uint32_t cap, uint32_t &poff, uint32_t &seg)
 sph_status run_emit(sph_ctx *c)
 {
     if (c->emit_h.empty()) return SPH_OK;
+    // without valid keys the hash that follows counts the new particles with the others
+    const sph::CellCount none{nullptr, nullptr};
     sph::launch_emit(c->emit_d, (uint32_t) c->emit_h.size(), c->table_d, c->soa(c->cur, c->id_cur), c->key_h,
-                     c->ref_order() ? c->ocell : nullptr, c->k.h, c->stream);
+                     c->keys_valid ? c->counts() : none, c->ref_order() ? c->ocell : nullptr, c->k.h, c->stream);
     c->counts_stale = true;
     return launch_error("emitter launch");
 }
@@ -687,9 +744,9 @@ sph_status run_grid_reference(sph_ctx *c)
     return SPH_OK;
 }
 
-// Grid phase: hash (unless the previous integrate already did), stable LSD radix
-// sort of (cell, slot) -- or the reference's buckets -- cell start table, and
-// gather into sorted order.
+// Grid phase: hash (unless the previous integrate already did), then the cell table,
+// the stable sort by cell -- by counts or by digits, or the reference's buckets --
+// and the particles in that order.
 sph_status run_grid(sph_ctx *c)
 {
     const uint32_t n = c->nslots;
@@ -698,24 +755,39 @@ sph_status run_grid(sph_ctx *c)
     if (!c->keys_valid) {
         StageTimer t(c, SPH_STAGE_HASH);
         if (t.st) return t.st;
-        sph::launch_hash(cur, c->key_h, tab, c->k.h, c->stream);
+        sph::launch_hash(cur, c->key_h, c->counts(), tab, c->k.h, c->stream);
     }
-    if (c->ref_order()) {
-        SPH_TRY(run_grid_reference(c));
-    } else {
+    sph::ParticleSoA dst = c->soa(1 - c->cur, 1 - c->id_cur);
+    if (c->by_counts) {
+        {
+            StageTimer t(c, SPH_STAGE_CELLS);
+            if (t.st) return t.st;
+            sph::launch_cell_table(c->counts(), c->scan_state, c->cstart, c->total_cells, c->stream, c->scan_poll_limit);
+        }
         {
             StageTimer t(c, SPH_STAGE_SORT);
             if (t.st) return t.st;
-            radix_sort(c, c->key_h, nullptr, c->tiles_d, (uint32_t) c->tiles_h.size(), c->sort_bits);
+            sph::launch_place(c->key_h, c->counts(), c->scan_state, c->cstart, c->total_cells, c->key_t, c->key_s, tab,
+                              c->stream);
         }
-        StageTimer t(c, SPH_STAGE_CELLS);
-        if (t.st) return t.st;
-        sph::launch_cell_start(c->key_s, n, c->total_cells, c->cstart, c->stream);
-    }
-    {
         StageTimer t(c, SPH_STAGE_REORDER);
         if (t.st) return t.st;
-        sph::ParticleSoA dst = c->soa(1 - c->cur, 1 - c->id_cur);
+        sph::launch_gather(cur, dst, c->key_t, c->key_s, c->cstart, c->val_s, tab, c->stream);
+    } else {
+        if (c->ref_order()) {
+            SPH_TRY(run_grid_reference(c));
+        } else {
+            {
+                StageTimer t(c, SPH_STAGE_SORT);
+                if (t.st) return t.st;
+                radix_sort(c, c->key_h, nullptr, c->tiles_d, (uint32_t) c->tiles_h.size(), c->sort_bits);
+            }
+            StageTimer t(c, SPH_STAGE_CELLS);
+            if (t.st) return t.st;
+            sph::launch_cell_start(c->key_s, n, c->total_cells, c->cstart, c->stream);
+        }
+        StageTimer t(c, SPH_STAGE_REORDER);
+        if (t.st) return t.st;
         sph::launch_reorder(cur, dst, c->val_s, n, c->stream);
     }
     SPH_TRY(launch_error("grid phase launch"));
@@ -742,7 +814,7 @@ sph_status run_fused_tail(sph_ctx *c)
     const bool diag = (c->flags & SPH_FLAG_DIAGNOSTICS) != 0;
     sph::ParticleSoA in = c->soa(c->cur, c->id_cur);
     sph::ParticleSoA out = c->soa(1 - c->cur, c->id_cur);
-    sph::launch_forces_fused(in, c->key_s, c->cstart, c->fields(diag), c->nlists(), out, c->key_h,
+    sph::launch_forces_fused(in, c->key_s, c->cstart, c->fields(diag), c->nlists(), out, c->key_h, c->counts(),
                              diag ? c->acc[0] : nullptr, diag ? c->acc[1] : nullptr, diag ? c->acc[2] : nullptr,
                              c->table(), c->k, c->variant, c->ref_order(), c->stream);
     SPH_TRY(launch_error("fused forces launch"));
@@ -851,7 +923,8 @@ sph_status run_phase(sph_ctx *c, int phase)
         if (t.st) return t.st;
         sph::ParticleSoA in = c->soa(c->cur, c->id_cur);
         sph::ParticleSoA out = c->soa(1 - c->cur, c->id_cur);
-        sph::launch_integrate(in, c->acc[0], c->acc[1], c->acc[2], out, c->key_h, c->table(), c->k, c->stream);
+        sph::launch_integrate(in, c->acc[0], c->acc[1], c->acc[2], out, c->key_h, c->counts(), c->table(), c->k,
+                              c->stream);
         st = launch_error("integrate launch");
         if (!st) {
             c->cur = 1 - c->cur;
@@ -1209,8 +1282,10 @@ struct Snapshot {
         if (c->ocell) SPH_HIP(hipMemcpyAsync(c->ocell, m + 8 * P * 4, P * 4, hipMemcpyDeviceToDevice, c->stream));
         SPH_HIP(hipMemcpyAsync(c->table_d, table.data(), table.size() * sizeof(sph::Scene), hipMemcpyHostToDevice,
                                c->stream));
+        SPH_TRY(clear_counts(c));
         SPH_HIP(hipStreamSynchronize(c->stream));
-        c->keys_valid = keys_valid;
+        // the counts of the saved keys are gone: the next step hashes again
+        c->keys_valid = keys_valid && !c->by_counts;
         c->steps_done = steps_done;
         c->counts_stale = !c->emit_h.empty();
         return SPH_OK;

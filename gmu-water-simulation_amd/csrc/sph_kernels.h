@@ -95,14 +95,23 @@ constexpr int kNumVariants = 21;
 constexpr int kDefaultVariant = 12;  // 64 threads, 8 candidates, a 24-entry word queue: fastest measured on the 1M dam break
 extern const NeighbourVariant kNeighbourVariants[kNumVariants];
 
+// The grid phase's counts (canonical order): count[c] slots have cell c as their
+// key, and arr[i] is slot i's number among them, in no particular order. The
+// kernels that write keys also count (count == nullptr: they do not): live slots
+// one by one, a scene's unused slots (its dead cell) together.
+struct CellCount {
+    uint32_t *count;
+    uint32_t *arr;
+};
+
 // Emitters (one workgroup each) add particles at the start of a step and update
 // the live counts in the device scene table.
-void launch_emit(const Emitter *em, uint32_t nem, Scene *scenes, const ParticleSoA &p, uint32_t *key, uint32_t *ocell,
-                 double h, hipStream_t st);
+void launch_emit(const Emitter *em, uint32_t nem, Scene *scenes, const ParticleSoA &p, uint32_t *key, const CellCount &cc,
+                 uint32_t *ocell, double h, hipStream_t st);
 
 // Cell key of every slot below t.nslots: the hash of src/CCPUParticleSimulator.cpp:46-69
 // for live particles, the scene's dead cell for unused slots.
-void launch_hash(const ParticleSoA &p, uint32_t *key, const SceneTable &t, double h, hipStream_t st);
+void launch_hash(const ParticleSoA &p, uint32_t *key, const CellCount &cc, const SceneTable &t, double h, hipStream_t st);
 
 // A tile of the radix sort: up to kSortTile slots [start, start + count) of one
 // segment (a scene or a free range) whose cells start at coff. The digits are
@@ -175,6 +184,22 @@ void launch_ref_place(const RefBuffers &r, const uint32_t *skey, const uint32_t 
 void launch_ref_final(const RefBuffers &r, const uint32_t *gnew, const uint32_t *start, uint32_t *skey, uint32_t *perm,
                       uint32_t *ocell, const SceneTable &t, hipStream_t st);
 
+// The grid phase from the keys and their counts (canonical order), in three steps.
+// 1. The cell table, the counts' exclusive scan: start[c] = the first sorted slot
+//    of cell c, c in [0, ncells]. state: 8-byte words, scan_state_words(ncells) of
+//    them, zero before the first call.
+// 2. Every slot to its cell's range, in no particular order (list), and the sorted
+//    keys; the counts and the state are zeroed for the next step.
+// 3. The particles to their places, a stable sort by key, and the permutation.
+// Nothing is written for unused slots in 2 and 3.
+inline uint32_t scan_state_words(uint32_t ncells) { return scan_blocks(ncells + 1) + 1; }
+void launch_cell_table(const CellCount &cc, unsigned long long *state, uint32_t *start, uint32_t ncells, hipStream_t st,
+                       uint32_t poll_limit = kScanPollLimit);
+void launch_place(const uint32_t *key, const CellCount &cc, unsigned long long *state, const uint32_t *start,
+                  uint32_t ncells, uint32_t *list, uint32_t *skey, const SceneTable &t, hipStream_t st);
+void launch_gather(const ParticleSoA &src, const ParticleSoA &dst, const uint32_t *list, const uint32_t *skey,
+                   const uint32_t *start, uint32_t *perm, const SceneTable &t, hipStream_t st);
+
 // start[c] = first slot whose sorted key is >= c, c in [0, ncells].
 void launch_cell_start(const uint32_t *sorted_keys, uint32_t n, uint32_t ncells, uint32_t *start,
                        hipStream_t st);
@@ -204,13 +229,13 @@ void launch_collide(const ParticleSoA &p, float *ax, float *ay, float *az, const
 
 // Integrate from acc into out and hash the new positions into key_next (the integrate phase).
 void launch_integrate(const ParticleSoA &p, const float *ax, const float *ay, const float *az,
-                      const ParticleSoA &out, uint32_t *key_next, const SceneTable &t, const Consts &k,
-                      hipStream_t st);
+                      const ParticleSoA &out, uint32_t *key_next, const CellCount &cc, const SceneTable &t,
+                      const Consts &k, hipStream_t st);
 
 // Fused forces + walls + integrate + next hash. acc pointers may be null (then not stored).
 void launch_forces_fused(const ParticleSoA &p, const uint32_t *cell, const uint32_t *start,
                          const DensityFields &f, const NeighbourList &nl, const ParticleSoA &out,
-                         uint32_t *key_next, float *ax, float *ay, float *az, const SceneTable &t, const Consts &k,
-                         int variant, bool ref, hipStream_t st);
+                         uint32_t *key_next, const CellCount &cc, float *ax, float *ay, float *az,
+                         const SceneTable &t, const Consts &k, int variant, bool ref, hipStream_t st);
 
 }  // namespace sph

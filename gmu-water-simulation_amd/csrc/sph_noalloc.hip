@@ -201,7 +201,7 @@ sph_status step_noalloc(const sph_params *prm, const sph_device_state *st, uint3
     SPH_NOALLOC_TRY(check_launch("set-up launch"));
     const int passes = (key_bits(s.ncells) + kRadixBits - 1) / kRadixBits;   // keys up to the dead cell ncells
     int cur = 0, idc = 0;
-    launch_hash(soa(cur, idc), key_h, tab, k.h, stream);
+    launch_hash(soa(cur, idc), key_h, CellCount{nullptr, nullptr}, tab, k.h, stream);
     for (uint32_t step = 0; step < nsteps; ++step) {
         // grid phase: stable radix sort of (cell, slot), cell table, gather (as run_grid)
         const uint32_t *kin = key_h, *vin = nullptr;
@@ -219,8 +219,8 @@ sph_status step_noalloc(const sph_params *prm, const sph_device_state *st, uint3
         idc = 1 - idc;
         // density, then forces + walls + integrate + the next step's keys
         launch_density(soa(cur, idc), key_s, cstart, f, nl, tab, k, kDefaultVariant, false, stream);
-        launch_forces_fused(soa(cur, idc), key_s, cstart, f, nl, soa(1 - cur, idc), key_h, nullptr, nullptr, nullptr,
-                            tab, k, kDefaultVariant, false, stream);
+        launch_forces_fused(soa(cur, idc), key_s, cstart, f, nl, soa(1 - cur, idc), key_h, CellCount{nullptr, nullptr},
+                            nullptr, nullptr, nullptr, tab, k, kDefaultVariant, false, stream);
         cur = 1 - cur;
         SPH_NOALLOC_TRY(check_launch("step launch"));
     }

@@ -1,0 +1,100 @@
+"""The grid phase's stable sort by cell, where its parts change: cell counts at the
+edges of the scan's tiles (4,096 entries), slot counts at the edges of the
+workgroups (256), crowded cells, particles outside the box, and keys counted by the
+hash as well as by the step before. Against numpy's stable argsort of the cells."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def positions(layout, n, box, rng):
+    pos = (rng.random((n, 3)) - 0.5) * box
+    if layout == "one cell":
+        pos[:] = 0.001 * rng.random((n, 3))
+    elif layout == "two cells":
+        pos[:] = 0.001 * rng.random((n, 3))
+        pos[::2, 0] += 0.0914
+    elif layout == "outside":
+        pos[::3] *= 1e3
+        pos[1::7] = np.nan
+    return pos.astype(np.float32)
+
+
+def check_sorted(sim, lib, ncells):
+    pre = sim.debug(lib.DEBUG_CELL_PRESORT)
+    want = np.argsort(pre, kind="stable").astype(np.uint32)
+    np.testing.assert_array_equal(sim.debug(lib.DEBUG_PERM), want)
+    np.testing.assert_array_equal(sim.debug(lib.DEBUG_CELL), pre[want])
+    np.testing.assert_array_equal(sim.debug(lib.DEBUG_CELL_START),
+                                  np.searchsorted(pre[want], np.arange(ncells + 1), side="left").astype(np.uint32))
+    return pre, want
+
+
+@pytest.mark.parametrize("res,n,layout", [
+    ((1, 1, 1), 1, "uniform"), ((3, 5, 7), 255, "uniform"), ((3, 5, 7), 256, "uniform"), ((3, 5, 7), 257, "uniform"),
+    ((2, 23, 89), 5000, "uniform"),      # 4,094 cells: 4,096 scanned entries, one tile
+    ((3, 5, 273), 5000, "uniform"),      # 4,095: one entry of a second tile
+    ((16, 16, 16), 5000, "uniform"), ((65, 64, 63), 70000, "uniform"),   # 64 tiles; 1 more than a look-back reads
+    ((9, 9, 9), 3000, "one cell"), ((9, 9, 9), 4097, "two cells"), ((9, 8, 7), 3000, "outside"),
+    ((210, 200, 204), 3000, "uniform"),  # more cells than are worth counting: sorted by digits
+])
+def test_stable_sort_and_cell_table(hip, res, n, layout):
+    lib = hip._lib
+    h = float(hip.scenes.H)
+    box = np.array([(r - 0.5) * h for r in res], np.float32)
+    rng = np.random.default_rng([n, *res])
+    pos = positions(layout, n, box, rng)
+    vel = rng.normal(0, 0.5, (n, 3)).astype(np.float32)
+    print("grid %s, %d particles, %s" % (res, n, layout), flush=True)
+    sim = hip.HIPGridParticleSimulator(box, capacity=n + 300)   # unused slots after the particles
+    sim.upload(pos, vel)
+    dims, ncells = sim.grid_dims()
+    assert dims == res
+    sim.updateGrid()
+    pre, want = check_sorted(sim, lib, ncells)
+    p, v, ids = sim.download(by_id=False)
+    assert np.array_equal(ids, want)
+    assert np.array_equal(p.view(np.uint32), pos[want].view(np.uint32))
+    assert np.array_equal(v.view(np.uint32), vel[want].view(np.uint32))
+    # the next sort starts from the keys that the integration wrote
+    sim.updateDensityPressure()
+    sim.updateForces()
+    sim.updateCollisions()
+    sim.integrate()
+    sim.updateGrid()
+    check_sorted(sim, lib, ncells)
+    for phase in (sim.updateDensityPressure, sim.updateForces, sim.updateCollisions, sim.integrate):
+        phase()
+    # and from those that the fused step wrote
+    sim.advance(2)
+    sim.updateGrid()
+    check_sorted(sim, lib, ncells)
+    sim.close()
+
+
+def test_sort_with_uneven_scenes_and_an_emitter(hip):
+    """Scenes with unused slots, an empty one and one that grows on the device: in
+    every scene the cell table counts exactly the live particles, step after step,
+    eagerly and from graphs."""
+    lib = hip._lib
+    for graphs in (False, True):
+        b = hip.SceneBatch([(0.4, 700), (0.3, 600), (0.5, 2000)])
+        rng = np.random.default_rng(7)
+        b.upload(0, ((rng.random((650, 3)) - 0.5) * 0.4).astype(np.float32))
+        b.upload(2, ((rng.random((900, 3)) - 0.5) * 0.5).astype(np.float32))
+        b.set_emitter(2, rate=150, limit=1900, radius=0.1, seed=5)
+        b.set_graphs(graphs)
+        for step in range(6):
+            b.phase(lib.PHASE_GRID)
+            for i, n in ((0, 650), (1, 0), (2, min(1900, 900 + 150 * (3 * step + 1)))):
+                assert b.count(i) == n
+                cells = b.debug(i, lib.DEBUG_CELL)
+                start = b.debug(i, lib.DEBUG_CELL_START)
+                want = np.searchsorted(cells, np.arange(len(start)), side="left").astype(np.uint32)
+                assert np.all(np.diff(cells.astype(np.int64)) >= 0) and np.array_equal(start, want)
+                assert np.array_equal(np.sort(b.download(i, by_id=False)[2]), np.arange(n))
+            for phase in (lib.PHASE_DENSITY, lib.PHASE_FORCES, lib.PHASE_COLLISIONS, lib.PHASE_INTEGRATE):
+                b.phase(phase)
+            b.step(2)
+        b.close()
