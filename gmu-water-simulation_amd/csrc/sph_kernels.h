@@ -76,7 +76,7 @@ constexpr int kSortTile = kSortThreads * kSortItems;
 constexpr int kScanTile = 4096;  // elements per 1024-thread scan block
 
 inline uint32_t sort_blocks(uint32_t n) { return (n + kSortTile - 1) / kSortTile; }
-inline uint32_t scan_blocks(uint32_t m) { return (m + kScanTile - 1) / kScanTile; }
+__host__ __device__ inline uint32_t scan_blocks(uint32_t m) { return (m + kScanTile - 1) / kScanTile; }
 
 // The tunable shape of the two neighbour kernels: workgroup size, candidates
 // tested per lane per trip, and how the force pass reads the row masks: with
@@ -192,7 +192,7 @@ void launch_ref_final(const RefBuffers &r, const uint32_t *gnew, const uint32_t 
 //    keys; the counts and the state are zeroed for the next step.
 // 3. The particles to their places, a stable sort by key, and the permutation.
 // Nothing is written for unused slots in 2 and 3.
-inline uint32_t scan_state_words(uint32_t ncells) { return scan_blocks(ncells + 1) + 1; }
+__host__ __device__ inline uint32_t scan_state_words(uint32_t ncells) { return scan_blocks(ncells + 1) + 1; }
 void launch_cell_table(const CellCount &cc, unsigned long long *state, uint32_t *start, uint32_t ncells, hipStream_t st,
                        uint32_t poll_limit = kScanPollLimit);
 void launch_place(const uint32_t *key, const CellCount &cc, unsigned long long *state, const uint32_t *start,

@@ -147,8 +147,8 @@ sph_status sph_step(sph_ctx *ctx, uint32_t nsteps, float *ms_out);
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc):
  * the steps of sph_step on particle arrays the caller owns in device memory, calling no
  * hipMalloc/hipFree or other allocating routine. Every other buffer (the second particle
- * buffer, sort keys and permutation, radix histograms, the cell table, density records)
- * lives in one static device array of SPH_NOALLOC_SCRATCH_BYTES per GPU, held until the
+ * buffer, sort keys and permutation, the cells' counts and table, density records, row
+ * masks) lives in one static device array of SPH_NOALLOC_SCRATCH_BYTES per GPU, held until the
  * process ends. `state` holds n particles in array order (structure of arrays, device
  * pointers); params gives box, gravity and dt (capacity, flags and max_neighbours are
  * not used). The call enqueues nsteps steps on `stream` (a hipStream_t; NULL = the null
@@ -159,7 +159,7 @@ sph_status sph_step(sph_ctx *ctx, uint32_t nsteps, float *ms_out);
  * calls that overlap on one GPU (other threads or streams) race and must not be made. */
 #define SPH_NOALLOC_MAX_PARTICLES 65536u
 #define SPH_NOALLOC_MAX_CELLS 262144u
-#define SPH_NOALLOC_SCRATCH_BYTES 7357696u
+#define SPH_NOALLOC_SCRATCH_BYTES 46138880u
 typedef struct {
     float *px, *py, *pz;
     float *vx, *vy, *vz;
