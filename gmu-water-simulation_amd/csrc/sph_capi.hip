@@ -112,6 +112,7 @@ struct sph_ctx {
     unsigned long long *scan_state = nullptr;
     uint32_t ccount_cap = 0;
     bool by_counts = false;   // the layout's grid phase sorts by counts (else by digits)
+    bool split = false;       // its neighbour passes share a particle between lanes (mask mode)
     uint32_t *hist = nullptr;
     uint32_t *partials = nullptr;
     uint32_t *cstart = nullptr;
@@ -180,7 +181,7 @@ struct sph_ctx {
         nl.idx = nlist;
         nl.cnt = nlist_cnt;
         nl.kmax = kmax;
-        nl.mode = nb_mode;
+        nl.mode = nb_mode == SPH_NEIGHBOURS_MASKS && split ? (int) sph::kNbSplit : nb_mode;
         nl.masks = masks;
         return nl;
     }
@@ -557,6 +558,9 @@ sph_status rebuild_layout(sph_ctx *c)
         SPH_TRY(dalloc(c, &c->cstart, want));
         c->cstart_cap = want;
     }
+    uint32_t widest = 0;
+    for (const sph::Scene &seg : c->table_h) widest = std::max(widest, seg.ncells ? seg.cap : 0u);
+    c->split = sph::split_neighbours(c->nslots, widest);
     c->by_counts = !c->ref_order() && sort_by_counts(c->total_cells, c->nslots);
     if (c->by_counts && c->total_cells + 1 > c->ccount_cap) {
         dfree(c, c->ccount);

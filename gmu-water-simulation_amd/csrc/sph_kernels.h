@@ -36,7 +36,11 @@ struct DensityFields {
 //
 // Or (mode kNbMasks) the density pass's per-row accepted-candidate masks
 // (`masks`, see the kernels), with cnt[i] = 1 for a particle they cannot hold.
-enum NeighbourMode : int { kNbWalk = 0, kNbLists = 1, kNbMasks = 2 };
+//
+// Or, in place of kNbMasks for launches that split_neighbours picks (kNbSplit), the
+// neighbours as 16-bit slots in the masks' words, kSplitCap at most, cnt[i] their
+// number or kNbOverflow for a particle with more.
+enum NeighbourMode : int { kNbWalk = 0, kNbLists = 1, kNbMasks = 2, kNbSplit = 3 };
 
 constexpr uint32_t kRecWords = 10;
 
@@ -48,6 +52,21 @@ constexpr uint32_t kRecWords = 10;
 constexpr uint32_t kMaskWordBits = 32;
 constexpr uint32_t kMaskWords = 16;
 constexpr uint32_t kMaskBits = kMaskWordBits * kMaskWords;
+
+constexpr uint32_t kSplitCap = 2u * 9u * kMaskWords;
+constexpr uint32_t kNbOverflow = 0xFFFFFFFFu;
+
+// Whether the neighbour passes of a launch over `slots` slots, the widest scene of
+// `widest`, share each particle between four lanes (k_density_split, k_forces_split):
+// faster while one wave's time decides, slower once there are waves enough to fill the
+// vector units, which the shared density pass uses less well. A step of one scene from
+// graphs, us, shared and not: dams of 500 particles 36 and 54, 4,096 44 and 60, 16,000 65
+// and 76, 32,000 84 and 89, 50,000 105 and 97; pools of 32,000 67 and 77, 50,000 91 and
+// 83; four scenes of 16,000 96 and 82. (Entries are 16-bit slots.)
+inline bool split_neighbours(uint32_t slots, uint32_t widest)
+{
+    return widest <= 65536u && slots <= 40960u;
+}
 
 struct NeighbourList {
     uint32_t *idx;

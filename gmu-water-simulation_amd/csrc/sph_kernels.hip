@@ -1162,6 +1162,27 @@ __device__ __forceinline__ float spiky_scale(double hr, float r2, const Consts &
     return spiky_factor(hr, r2, k.spiky, g_pow2_exc, g_pow2_exc_count);
 }
 
+// The density results of a particle: density, and the
+// force pass's record with p/rho^2 (double, as src/CCPUParticleSimulator.cpp:181
+// forms it) and 1/rho (double).
+__device__ __forceinline__ void store_density(const DensityFields &f, const ParticleSoA &p, const Consts &k, uint32_t i,
+                                              float density, float xi, float yi, float zi)
+{
+    const float pressure = k.gas_k * (density - k.rho0);
+    f.rho[i] = density;
+    // rho*rho is exact in double, so this is p / pow(rho, 2)
+    const double prr = (double) pressure / ((double) density * (double) density);
+    const double rinv = 1.0 / (double) density;
+    // the record, as five 8-byte stores (records are 8-byte aligned)
+    uint2 *rec = reinterpret_cast<uint2 *>(f.rec + kRecWords * (size_t) i);
+    const uint64_t pb = __builtin_bit_cast(uint64_t, prr), rb = __builtin_bit_cast(uint64_t, rinv);
+    rec[0] = make_uint2(__float_as_uint(xi), __float_as_uint(yi));
+    rec[1] = make_uint2(__float_as_uint(zi), __float_as_uint(p.vx[i]));
+    rec[2] = make_uint2(__float_as_uint(p.vy[i]), __float_as_uint(p.vz[i]));
+    rec[3] = make_uint2((uint32_t) pb, (uint32_t) (pb >> 32));
+    rec[4] = make_uint2((uint32_t) rb, (uint32_t) (rb >> 32));
+}
+
 // updateDensityPressure, src/CCPUParticleSimulator.cpp:93-141. Also stores
 // p/rho^2 (double, as src/CCPUParticleSimulator.cpp:181 forms it), 1/rho
 // (double) and, for the force pass, with kLists the particle's accepted
@@ -1225,19 +1246,7 @@ __global__ __launch_bounds__(T) void k_density(ParticleSoA p, const uint32_t *__
     else
         walk_neighbours<kRef, U, false, kCap>(s, k, start, bv, x, y, z, xi, yi, zi, cnt, test, flush);
     density = density * k.mass;
-    const float pressure = k.gas_k * (density - k.rho0);
-    f.rho[i] = density;
-    // rho*rho is exact in double, so this is p / pow(rho, 2)
-    const double prr = (double) pressure / ((double) density * (double) density);
-    const double rinv = 1.0 / (double) density;
-    // the record, as five 8-byte stores (records are 8-byte aligned)
-    uint2 *rec = reinterpret_cast<uint2 *>(f.rec + kRecWords * (size_t) i);
-    const uint64_t pb = __builtin_bit_cast(uint64_t, prr), rb = __builtin_bit_cast(uint64_t, rinv);
-    rec[0] = make_uint2(__float_as_uint(xi), __float_as_uint(yi));
-    rec[1] = make_uint2(__float_as_uint(zi), __float_as_uint(p.vx[i]));
-    rec[2] = make_uint2(__float_as_uint(p.vy[i]), __float_as_uint(p.vz[i]));
-    rec[3] = make_uint2((uint32_t) pb, (uint32_t) (pb >> 32));
-    rec[4] = make_uint2((uint32_t) rb, (uint32_t) (rb >> 32));
+    store_density(f, p, k, i, density, xi, yi, zi);
     if (kLists) nl.cnt[i] = nn;
     if (kMasks) nl.cnt[i] = rec_masks.overflow ? 1u : 0u;
     if (kDiag) f.ncount[i] = nc;
@@ -1818,6 +1827,236 @@ __global__ __launch_bounds__(T) void k_forces_fused(ParticleSoA p, const uint32_
     if (!kRef && cc.count) count_key(cc, i, c);
 }
 
+// ---------------------------------------------------------------- neighbour passes of small launches
+//
+// With one lane a particle, a launch of a few hundred waves leaves most SIMDs with
+// one wave or none, and takes as long as its longest wave, a wave alone issuing a vector
+// instruction every 7 cycles or so. Here four lanes share a particle, 16 particles a
+// wave, and the particle's terms are still added in the canonical order: at 4,096
+// particles 25.9 -> 17.4 us for the density and 19.2 -> 9.2 us for the force pass, at
+// 50,653 no longer (51 -> 77 and 39 -> 23 us), and at 1,048,576 the shared force pass
+// has half as much again of vector instructions (357 -> 486 us).
+
+// The density pass for small launches. Lane 16g + p of a wave tests the candidates of
+// some of particle p's 9 rows, in order (rows 2g and 2g + 1; the last lane also row
+// 8), and lists the accepted ones in LDS; a full lane waits. When no lane can go on,
+// the first lane of each particle adds the lists in order, up to the first lane that
+// is not through its rows yet: it always is when that lane is the first unfinished
+// one, so the lists empty and the wait ends. It also writes the particle's neighbours
+// (minus itself) to its neighbour list for the force pass: 16-bit slots, kSplitCap of
+// them in the masks' words (more: cnt = kNbOverflow), entry e of slot i at
+// e * 64 + i % 64 of its block of 64 slots.
+constexpr int kSplitCand = 8;    // candidates a lane tests per trip
+constexpr int kSplitList = 32;   // accepted candidates a lane holds
+
+__device__ __forceinline__ uint16_t *split_list(uint32_t *masks, uint32_t i)
+{
+    return reinterpret_cast<uint16_t *>(masks + (size_t) (i >> 6) * (9u * kMaskWords * 64u)) + (i & 63u);
+}
+static_assert(kSplitCap * 64u * 2u <= 9u * kMaskWords * 64u * 4u, "the lists fit the masks' words");
+
+template <bool kDiag, bool kRef>
+__global__ __launch_bounds__(64) void k_density_split(ParticleSoA p, const uint32_t *__restrict__ cell,
+                                                      const uint32_t *__restrict__ start, DensityFields f,
+                                                      NeighbourList nl, SceneTable t, Consts k)
+{
+    __shared__ float s_r2[kSplitList * 64];
+    __shared__ uint16_t s_j[kSplitList * 64];
+    __shared__ uint32_t s_state[64];   // accepted candidates in a lane's list, and (bit 31) whether its rows are done
+    const uint32_t lane = threadIdx.x, sub = lane & 15u, g = lane >> 4;
+    const uint32_t first = xcd_block(blockIdx.x, gridDim.x) * 16u, i = first + sub;
+    const Scene s = block_scene(t, first);
+    if (first - s.poff >= s.n) return;
+    const uint32_t li = i - s.poff;
+    const bool live = li < s.n;
+    const BufView bv = buf_view(p, f, s);
+    const float xi = ldf(bv.px, li * 4u), yi = ldf(bv.py, li * 4u), zi = ldf(bv.pz, li * 4u);
+    int x = 0, y = 0, z = 0;
+    if (live) cell_xyz<kRef>(cell[i], s, x, y, z);
+    const RowBounds rb = row_bounds(s, k, x, y, z, xi, yi, zi);
+    int r = (int) (2u * g);
+    const int rlast = g == 3u ? 8 : r + 1;
+    uint32_t j = 0, jend = 0;
+    if (live) row_run<kRef>(rb, s, start, x, y, z, r, j, jend);
+    bool done = !live;
+    int cnt = 0;
+    // the particle's sum, in its first lane; nn: neighbours listed, nc: accepted, gcur: the list at hand
+    float density = 0.0f;
+    uint32_t nn = 0, nc = 0, gcur = live ? 0u : 4u;
+    uint16_t *lst = split_list(nl.masks, i);
+    for (;;) {
+        for (;;) {
+            const bool full = cnt > kSplitList - kSplitCand;
+            if (!done && j >= jend) {
+                if (r == rlast) {
+                    done = true;
+                } else {
+                    ++r;
+                    row_run<kRef>(rb, s, start, x, y, z, r, j, jend);
+                }
+            }
+            if (!__any(!done && !full)) break;
+            if (j < jend && !full) {
+                const uint32_t off = j * 4u, rem = jend - j;
+                float cx[kSplitCand], cy[kSplitCand], cz[kSplitCand];
+#pragma unroll
+                for (int u = 0; u < kSplitCand; ++u) {
+                    cx[u] = ldf(bv.px, off + 4u * u);
+                    cy[u] = ldf(bv.py, off + 4u * u);
+                    cz[u] = ldf(bv.pz, off + 4u * u);
+                }
+#pragma unroll
+                for (int u = 0; u < kSplitCand; ++u) {
+                    const float dx = xi - cx[u], dyv = yi - cy[u], dzv = zi - cz[u];
+                    const float r2 = dx * dx + dyv * dyv + dzv * dzv;
+                    s_r2[cnt * 64 + lane] = r2;
+                    s_j[cnt * 64 + lane] = (uint16_t) (j + u);
+                    cnt += ((uint32_t) u < rem) & (r2 <= k.hsq_f);
+                }
+                j += kSplitCand;
+            }
+        }
+        s_state[lane] = (uint32_t) cnt | (done ? 0x80000000u : 0u);
+        __builtin_amdgcn_wave_barrier();
+        if (lane < 16u) {
+            while (gcur < 4u) {
+                const uint32_t at = gcur * 16u + sub, st = s_state[at], c = st & 0x7FFFFFFFu;
+                auto list = [&](uint32_t e) {
+                    const uint32_t jj = s_j[e * 64u + at];
+                    if (jj != li) {
+                        if (nn < kSplitCap) lst[nn * 64u] = (uint16_t) jj;
+                        ++nn;
+                    }
+                };
+                uint32_t e = 0;
+                for (; e + 1u < c; e += 2u) {
+                    const float ra = s_r2[e * 64u + at], rb2 = s_r2[(e + 1u) * 64u + at];
+                    const double ta = k.hsq - (double) ra, tb = k.hsq - (double) rb2;
+                    const double pa = density_poly(ta, k.poly6), pb = density_poly(tb, k.poly6);
+                    density = density_accumulate(density, pa, ta, ra, k.poly6, g_pow3_exc, g_pow3_exc_count);
+                    density = density_accumulate(density, pb, tb, rb2, k.poly6, g_pow3_exc, g_pow3_exc_count);
+                    list(e);
+                    list(e + 1u);
+                }
+                if (e < c) {
+                    density = density_add(density, s_r2[e * 64u + at], k);
+                    list(e);
+                }
+                nc += c;
+                s_state[at] = st & 0x80000000u;
+                if (!(st >> 31)) break;
+                ++gcur;
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+        cnt = (int) (s_state[lane] & 0x7FFFFFFFu);
+        if (!__any(lane < 16u && gcur < 4u)) break;
+    }
+    if (lane >= 16u || !live) return;
+    density = density * k.mass;
+    store_density(f, p, k, i, density, xi, yi, zi);
+    nl.cnt[i] = nn <= kSplitCap ? nn : kNbOverflow;
+    if (kDiag) f.ncount[i] = nc;
+}
+
+// The value of lane Q of each four lanes.
+template <int Q>
+__device__ __forceinline__ float quad_lane(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), Q * 0x55, 0xf, 0xf, true));
+}
+
+// The forces of 16 particles a wave from the neighbour lists of k_density_split: lane
+// 4p + q computes the terms of particle p's neighbours q, q + 4, ..., and every four
+// are added in order, by all four lanes alike (a lane without a pair adds +0, which
+// leaves a sum as it is: sums start at +0 and are never -0). kFused: walls,
+// integration and the next keys, as k_forces_fused; else the acceleration alone.
+template <bool kFused, bool kStoreAcc, bool kRef>
+__global__ __launch_bounds__(64) void k_forces_split(ParticleSoA p, const uint32_t *__restrict__ cell,
+                                                     const uint32_t *__restrict__ start, DensityFields f,
+                                                     NeighbourList nl, ParticleSoA out,
+                                                     uint32_t *__restrict__ key_next, CellCount cc,
+                                                     float *__restrict__ ax, float *__restrict__ ay,
+                                                     float *__restrict__ az, SceneTable t, Consts k)
+{
+    __shared__ uint32_t lst[kListCap * 64];
+    const uint32_t lane = threadIdx.x, q = lane & 3u;
+    const uint32_t first = xcd_block(blockIdx.x, gridDim.x) * 16u, i = first + (lane >> 2);
+    const Scene s = block_scene(t, first);
+    const uint32_t li = i - s.poff;
+    if (i >= t.nslots) return;
+    if (kFused && !kRef && q == 0u) count_dead(cc, i, s);
+    if (li >= s.n) {
+        if (kFused && q == 0u) key_next[i] = dead_key(s);
+        return;
+    }
+    const BufView bv = buf_view(p, f, s);
+    const float xi = p.px[i], yi = p.py[i], zi = p.pz[i];
+    const float vxi = p.vx[i], vyi = p.vy[i], vzi = p.vz[i];
+    const float rhoi = f.rho[i];
+    const double ai = own_prr(f, i);
+    const uint32_t cnt_i = nl.cnt[i];
+    ForceSums a = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    if (cnt_i == kNbOverflow) {
+        a = walk_sums<kRef, 64, 4>(bv, cell, start, lst + lane, i, li, s, k, xi, yi, zi, vxi, vyi, vzi, ai);
+    } else {
+        const uint16_t *nb = split_list(nl.masks, i);
+        // loaded by lanes without a pair, never added (a record offset)
+        const uint32_t fallback = (li + 1 < s.n ? li + 1 : li - 1) * (4u * kRecWords);
+        auto offset = [&](uint32_t e) { return e < cnt_i ? (uint32_t) nb[e * 64u] * (4u * kRecWords) : fallback; };
+        auto add = [&](const PairData &n, bool have) {
+            PairTerms v = pair_terms(bv, k, n, xi, yi, zi, vxi, vyi, vzi, ai);
+            if (!have) v = PairTerms{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+#define SPH_QUAD_ADD(c) \
+    a.c = a.c + quad_lane<0>(v.c); \
+    a.c = a.c + quad_lane<1>(v.c); \
+    a.c = a.c + quad_lane<2>(v.c); \
+    a.c = a.c + quad_lane<3>(v.c)
+            SPH_QUAD_ADD(px);
+            SPH_QUAD_ADD(py);
+            SPH_QUAD_ADD(pz);
+            SPH_QUAD_ADD(vx);
+            SPH_QUAD_ADD(vy);
+            SPH_QUAD_ADD(vz);
+#undef SPH_QUAD_ADD
+        };
+        // the records of the next two rounds are in flight, and the list entries after them
+        PairData pa = load_pair_at(bv, offset(q)), pb = load_pair_at(bv, offset(q + 4u));
+        uint32_t oc = offset(q + 8u), od = offset(q + 12u);
+        for (uint32_t e = q; __any(e - q < cnt_i); e += 8u) {
+            const PairData pc = load_pair_at(bv, oc), pd = load_pair_at(bv, od);
+            oc = offset(e + 16u);
+            od = offset(e + 20u);
+            add(pa, e < cnt_i);
+            add(pb, e + 4u < cnt_i);
+            pa = pc;
+            pb = pd;
+        }
+    }
+    float a0, a1, a2;
+    accel_from_sums(a, rhoi, s, k, a0, a1, a2);
+    if (kFused) wall_accel(xi, yi, zi, vxi, vyi, vzi, s, k, a0, a1, a2);
+    if (kStoreAcc && q == 0u) {
+        ax[i] = a0;
+        ay[i] = a1;
+        az[i] = a2;
+    }
+    if (!kFused) return;
+    float nx, ny, nz, nvx, nvy, nvz;
+    integrate_one(xi, yi, zi, vxi, vyi, vzi, a0, a1, a2, s.dt, nx, ny, nz, nvx, nvy, nvz);
+    const uint32_t c = hash_key<kRef>(nx, ny, nz, s, k.h);
+    if (q == 0u) {
+        out.px[i] = nx; out.py[i] = ny; out.pz[i] = nz;
+        out.vx[i] = nvx; out.vy[i] = nvy; out.vz[i] = nvz;
+        key_next[i] = c;
+    }
+    if (!kRef && cc.count) {
+        // lane l counts for particle l (the live particles are the wave's first lanes' fours)
+        const uint32_t ck = (uint32_t) __shfl((int) c, (int) (4u * lane) & 63, 64);
+        if (lane < 16u && first + lane - s.poff < s.n) count_key(cc, first + lane, ck);
+    }
+}
+
 inline uint32_t blocks_for(uint32_t n, uint32_t t) { return (n + t - 1) / t; }
 
 // The compiled shapes of the two neighbour kernels, indexed by variant.
@@ -2060,6 +2299,25 @@ void launch_reorder(const ParticleSoA &src, const ParticleSoA &dst, const uint32
         hipLaunchKernelGGL(k_reorder<4>, dim3(blocks_for(n, 256 * 4)), dim3(256), 0, st, src, dst, perm, n);
 }
 
+// The split force pass: fused (accelerations stored if ax is given) or the phase.
+template <bool kFused>
+static void launch_forces_split(const ParticleSoA &p, const uint32_t *cell, const uint32_t *start,
+                                const DensityFields &f, const NeighbourList &nl, const ParticleSoA &out,
+                                uint32_t *key_next, const CellCount &cc, float *ax, float *ay, float *az,
+                                const SceneTable &t, const Consts &k, bool ref, hipStream_t st)
+{
+    const dim3 g(blocks_for(t.nslots, 16));
+#define SPH_SPLIT_FORCES(acc, ref_)                                                                                   \
+    hipLaunchKernelGGL((k_forces_split<kFused, acc, ref_>), g, dim3(64), 0, st, p, cell, start, f, nl, out, key_next, \
+                       cc, ax, ay, az, t, k)
+    if (ax) {
+        if (ref) SPH_SPLIT_FORCES(true, true); else SPH_SPLIT_FORCES(true, false);
+    } else if constexpr (kFused) {
+        if (ref) SPH_SPLIT_FORCES(false, true); else SPH_SPLIT_FORCES(false, false);
+    }
+#undef SPH_SPLIT_FORCES
+}
+
 // The reference order (kRef) is compiled in one shape, variant 12's.
 using RefKernels = NeighbourKernels<64, 8, 48, 0, true, true>;
 
@@ -2068,6 +2326,18 @@ void launch_density(const ParticleSoA &p, const uint32_t *cell, const uint32_t *
                     hipStream_t st)
 {
     if (t.nslots == 0) return;
+    if (nl.mode == kNbSplit) {
+        const dim3 g(blocks_for(t.nslots, 16));
+#define SPH_SPLIT_DENSITY(diag, ref_) \
+    hipLaunchKernelGGL((k_density_split<diag, ref_>), g, dim3(64), 0, st, p, cell, start, f, nl, t, k)
+        if (f.ncount) {
+            if (ref) SPH_SPLIT_DENSITY(true, true); else SPH_SPLIT_DENSITY(true, false);
+        } else {
+            if (ref) SPH_SPLIT_DENSITY(false, true); else SPH_SPLIT_DENSITY(false, false);
+        }
+#undef SPH_SPLIT_DENSITY
+        return;
+    }
     if (ref) {
         RefKernels::density(st, p, cell, start, f, nl, t, k);
         return;
@@ -2086,6 +2356,11 @@ void launch_forces(const ParticleSoA &p, const uint32_t *cell, const uint32_t *s
                    bool ref, hipStream_t st)
 {
     if (t.nslots == 0) return;
+    if (nl.mode == kNbSplit) {
+        launch_forces_split<false>(p, cell, start, f, nl, ParticleSoA{}, nullptr, CellCount{nullptr, nullptr}, ax, ay, az, t,
+                                   k, ref, st);
+        return;
+    }
     if (ref)
         hipLaunchKernelGGL(k_forces<true>, dim3(blocks_for(t.nslots, kPhaseThreads)), dim3(kPhaseThreads), 0, st, p,
                            cell, start, f, nl, ax, ay, az, t, k);
@@ -2115,6 +2390,10 @@ void launch_forces_fused(const ParticleSoA &p, const uint32_t *cell, const uint3
                          hipStream_t st)
 {
     if (t.nslots == 0) return;
+    if (nl.mode == kNbSplit) {
+        launch_forces_split<true>(p, cell, start, f, nl, out, key_next, cc, ax, ay, az, t, k, ref, st);
+        return;
+    }
     if (ref) {
         RefKernels::fused(st, p, cell, start, f, nl, out, key_next, cc, ax, ay, az, t, k);
         return;

@@ -177,7 +177,7 @@ sph_status step_noalloc(const sph_params *prm, const sph_device_state *st, uint3
     nl.idx = nullptr;
     nl.cnt = u32(kOffCnt);
     nl.kmax = 0;
-    nl.mode = kNbMasks;
+    nl.mode = split_neighbours(n, n) ? kNbSplit : kNbMasks;
     nl.masks = u32(kOffMasks);
     SceneTable tab{scene_d, nullptr, n};
     const Consts k = make_consts();
