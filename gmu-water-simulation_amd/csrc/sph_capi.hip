@@ -148,10 +148,17 @@ struct sph_ctx {
     bool use_graphs = false;
     hipGraphExec_t graph[2][2] = {};
 
-    // readback: pinned host buffers the device writes by id
+    // uploads: two pinned parts, each of up_cap particles' positions, velocities and ids;
+    // one is filled while the device reads the other
+    float *up[2] = {};
+    hipEvent_t up_read[2] = {};
+    uint32_t up_cap = 0;
+
+    // readback: pinned host buffers the device writes by id, its flag behind the
+    // positions, and (device) each id's slot
     float *rb_pos = nullptr, *rb_vel = nullptr;
     size_t rb_cap = 0;
-    uint32_t *rb_bad = nullptr;
+    uint32_t *rb_at = nullptr;
 
     // profiling
     hipEvent_t ev[kProfileSlots][2] = {};
@@ -311,11 +318,23 @@ void drop_graphs(sph_ctx *c)
             }
 }
 
+void free_upload(sph_ctx *c)
+{
+    for (int part = 0; part < 2; ++part) {
+        if (c->up[part]) (void) hipHostFree(c->up[part]);
+        if (c->up_read[part]) (void) hipEventDestroy(c->up_read[part]);
+        c->up[part] = nullptr;
+        c->up_read[part] = nullptr;
+    }
+    c->up_cap = 0;
+}
+
 void release(sph_ctx *c)
 {
     if (!c) return;
     if (c->stream) (void) hipStreamSynchronize(c->stream);
     drop_graphs(c);
+    free_upload(c);
     if (c->rb_pos) (void) hipHostFree(c->rb_pos);
     if (c->rb_vel) (void) hipHostFree(c->rb_vel);
     for (void *p : c->allocations) (void) hipFree(p);
@@ -951,36 +970,49 @@ sph_status copy_d2h(sph_ctx *c, void *dst, const void *src, size_t bytes)
     return SPH_OK;
 }
 
-sph_status copy_h2d(sph_ctx *c, void *dst, const void *src, size_t bytes)
+// Particles an upload's part holds: its copies stay in the processor's caches, and
+// reading one part takes the device longer than a launch.
+constexpr uint32_t kUploadPart = 16384;
+
+// The pinned parts, for uploads of n particles.
+sph_status ensure_upload(sph_ctx *c, uint32_t n)
 {
-    if (bytes == 0) return SPH_OK;
-    SPH_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
-    SPH_HIP(hipStreamSynchronize(c->stream));
+    const uint32_t want = round_up(std::min(n, kUploadPart), 256);
+    if (want <= c->up_cap) return SPH_OK;
+    free_upload(c);
+    for (int part = 0; part < 2; ++part) {
+        SPH_HIP(hipHostMalloc((void **) &c->up[part], (size_t) want * 28, hipHostMallocDefault));
+        SPH_HIP(hipEventCreateWithFlags(&c->up_read[part], hipEventDisableTiming));
+    }
+    c->up_cap = want;
     return SPH_OK;
 }
 
 // Writes n particles into slots first.. of the current buffers; ids default to
-// id_base + index.
+// id_base + index. Uploaded and appended particles join the back of cell (0,0,0)'s
+// bucket in the reference order (addParticle). The stream holds no upload on entry.
 sph_status write_slots(sph_ctx *c, const float *pos3, const float *vel3, const uint32_t *ids, uint32_t first,
                        uint32_t n, uint32_t id_base)
 {
     if (n == 0) return SPH_OK;
-    std::vector<float> buf((size_t) n);
-    std::vector<uint32_t> ib((size_t) n);
-    for (int comp = 0; comp < 3; ++comp) {
-        for (uint32_t i = 0; i < n; ++i) buf[i] = pos3[3 * (size_t) i + comp];
-        SPH_TRY(copy_h2d(c, c->pos[c->cur][comp] + first, buf.data(), n * sizeof(float)));
-        for (uint32_t i = 0; i < n; ++i) buf[i] = vel3 ? vel3[3 * (size_t) i + comp] : 0.0f;
-        SPH_TRY(copy_h2d(c, c->vel[c->cur][comp] + first, buf.data(), n * sizeof(float)));
+    SPH_TRY(ensure_upload(c, n));
+    sph_status st = SPH_OK;
+    for (uint32_t k = 0, q = 0; k < n && !st; k += c->up_cap, ++q) {
+        const int part = (int) (q & 1u);
+        const uint32_t m = std::min(c->up_cap, n - k);
+        if (q > 1) SPH_HIP(hipEventSynchronize(c->up_read[part]));
+        float *pos = c->up[part], *vel = pos + 3 * (size_t) c->up_cap;
+        uint32_t *id = (uint32_t *) (vel + 3 * (size_t) c->up_cap);
+        std::memcpy(pos, pos3 + 3 * (size_t) k, (size_t) m * 12);
+        if (vel3) std::memcpy(vel, vel3 + 3 * (size_t) k, (size_t) m * 12);
+        if (ids) std::memcpy(id, ids + k, (size_t) m * 4);
+        sph::launch_unpack(pos, vel3 ? vel : nullptr, ids ? id : nullptr, id_base + k, c->soa(c->cur, c->id_cur),
+                           c->ref_order() ? c->ocell : nullptr, first + k, m, c->stream);
+        st = launch_error("upload launch");
+        if (!st) SPH_HIP(hipEventRecord(c->up_read[part], c->stream));
     }
-    for (uint32_t i = 0; i < n; ++i) ib[i] = ids ? ids[i] : id_base + i;
-    SPH_TRY(copy_h2d(c, c->ids[c->id_cur] + first, ib.data(), n * sizeof(uint32_t)));
-    if (c->ref_order()) {
-        // uploaded and appended particles join the back of cell (0,0,0)'s bucket (addParticle)
-        std::fill(ib.begin(), ib.end(), 0u);
-        SPH_TRY(copy_h2d(c, c->ocell + first, ib.data(), n * sizeof(uint32_t)));
-    }
-    return SPH_OK;
+    SPH_HIP(hipStreamSynchronize(c->stream));
+    return st;
 }
 
 sph_status scene_write(sph_ctx *c, uint32_t scene, const float *pos3, const float *vel3, const uint32_t *ids,
@@ -1845,25 +1877,27 @@ sph_status sph_scene_readback(sph_ctx *c, uint32_t scene, int with_velocity, con
         SPH_TRY(sync_counts(c));
         const sph::Scene &s = c->scenes[scene].s;
         const uint32_t n = s.n;
-        if (n > c->rb_cap || (with_velocity && !c->rb_vel)) {
+        if (n > c->rb_cap || !c->rb_pos || (with_velocity && !c->rb_vel)) {
             SPH_HIP(hipStreamSynchronize(c->stream));
-            const size_t cap = std::max<size_t>(n, c->rb_cap);
+            const size_t cap = std::max<size_t>(std::max<size_t>(n, c->rb_cap), 1);
             if (c->rb_pos) (void) hipHostFree(c->rb_pos);
             if (c->rb_vel) (void) hipHostFree(c->rb_vel);
+            dfree(c, c->rb_at);
             c->rb_pos = c->rb_vel = nullptr;
+            c->rb_at = nullptr;
             c->rb_cap = 0;
-            SPH_HIP(hipHostMalloc((void **) &c->rb_pos, std::max<size_t>(cap, 1) * 12, hipHostMallocDefault));
-            if (with_velocity) SPH_HIP(hipHostMalloc((void **) &c->rb_vel, std::max<size_t>(cap, 1) * 12, hipHostMallocDefault));
+            SPH_HIP(hipHostMalloc((void **) &c->rb_pos, cap * 12 + 4, hipHostMallocDefault));
+            if (with_velocity) SPH_HIP(hipHostMalloc((void **) &c->rb_vel, cap * 12, hipHostMallocDefault));
+            SPH_TRY(dalloc(c, &c->rb_at, cap));
             c->rb_cap = cap;
         }
-        if (!c->rb_bad) SPH_TRY(dalloc(c, &c->rb_bad, 1));
-        SPH_HIP(hipMemsetAsync(c->rb_bad, 0, 4, c->stream));
-        sph::launch_scatter_by_id(c->soa(c->cur, c->id_cur), s.poff, n, c->rb_pos, with_velocity ? c->rb_vel : nullptr,
-                                  c->rb_bad, c->stream);
+        volatile uint32_t *bad = (volatile uint32_t *) (c->rb_pos + 3 * c->rb_cap);
+        *bad = 0;
+        sph::launch_pack_by_id(c->soa(c->cur, c->id_cur), s.poff, n, c->rb_at, c->rb_pos,
+                               with_velocity ? c->rb_vel : nullptr, (uint32_t *) bad, c->stream);
         SPH_TRY(launch_error("readback launch"));
-        uint32_t bad = 0;
-        SPH_TRY(copy_d2h(c, &bad, c->rb_bad, 4));
-        if (bad) return fail(SPH_ERR_STATE, "sph_scene_readback: particle ids are not 0..count-1");
+        SPH_HIP(hipStreamSynchronize(c->stream));
+        if (*bad) return fail(SPH_ERR_STATE, "sph_scene_readback: particle ids are not 0..count-1");
         *pos_xyz = c->rb_pos;
         if (vel_xyz) *vel_xyz = with_velocity ? c->rb_vel : nullptr;
         *count = n;

@@ -228,8 +228,10 @@ void launch_reorder(const ParticleSoA &src, const ParticleSoA &dst, const uint32
                     hipStream_t st);
 
 // pos[3*id + c] (and vel) for slots first .. first+n-1; ids outside 0..n-1 set *bad.
-void launch_scatter_by_id(const ParticleSoA &p, uint32_t first, uint32_t n, float *pos, float *vel, uint32_t *bad,
-                          hipStream_t st);
+void launch_unpack(const float *pos, const float *vel, const uint32_t *ids, uint32_t id_base, const ParticleSoA &p,
+                   uint32_t *ocell, uint32_t first, uint32_t n, hipStream_t st);
+void launch_pack_by_id(const ParticleSoA &p, uint32_t first, uint32_t n, uint32_t *at, float *pos, float *vel,
+                       uint32_t *bad, hipStream_t st);
 
 // Density pass: density, p/rho^2, 1/rho and the neighbour lists. `ref`: the
 // scenes use the reference order (kOrderReference; one kernel shape).

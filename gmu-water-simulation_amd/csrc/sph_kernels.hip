@@ -646,28 +646,98 @@ __global__ void k_reorder(ParticleSoA src, ParticleSoA dst, const uint32_t *__re
     }
 }
 
-// Particles first .. first+n-1 of the current order written by id into xyz
-// triples (render/readback order, as CGPUBaseParticleSimulator::integrate
-// un-permutes by id, src/CGPUBaseParticleSimulator.cpp:83-91). vel may be null.
-// An id outside 0..n-1 is not written; it raises *bad instead.
-__global__ __launch_bounds__(256) void k_scatter_by_id(ParticleSoA p, uint32_t first, uint32_t n,
-                                                       float *__restrict__ pos, float *__restrict__ vel,
-                                                       uint32_t *__restrict__ bad)
+// ---------------------------------------------------------------- particles in and out
+//
+// Host memory is read and written by the kernels, over the link, in whole 16-byte
+// pieces of consecutive addresses: it is the pinned xyz triples of 256 particles a
+// workgroup, turned into and out of the separate arrays in LDS. The link's 55 GB/s
+// bound them (24 MB of 1,048,576 particles' positions and velocities: 0.45 ms).
+
+constexpr uint32_t kTriples = 256;   // particles a workgroup
+
+// n particles from xyz triples in `pos` and `vel` (or at rest) and `ids` (or id_base,
+// id_base + 1, ...) into slots first .. first + n - 1; their cells become 0 in ocell, if
+// given. The host arrays are readable to a multiple of 4 words.
+__global__ __launch_bounds__(kTriples) void k_unpack(const float4 *__restrict__ pos, const float4 *__restrict__ vel,
+                                                     const uint32_t *__restrict__ ids, uint32_t id_base,
+                                                     ParticleSoA p, uint32_t *__restrict__ ocell, uint32_t first,
+                                                     uint32_t n)
+{
+    __shared__ float4 s_xyz[2][kTriples * 3 / 4];
+    const uint32_t k0 = blockIdx.x * kTriples, k = k0 + threadIdx.x;
+    const uint32_t words = 3u * (n - k0 < kTriples ? n - k0 : kTriples), pieces = (words + 3u) / 4u;
+    for (uint32_t q = threadIdx.x; q < pieces; q += kTriples) {
+        s_xyz[0][q] = pos[(size_t) blockIdx.x * (kTriples * 3 / 4) + q];
+        if (vel) s_xyz[1][q] = vel[(size_t) blockIdx.x * (kTriples * 3 / 4) + q];
+    }
+    __syncthreads();
+    if (k >= n) return;
+    const uint32_t i = first + k;
+    const float *x = reinterpret_cast<const float *>(s_xyz[0]) + 3u * threadIdx.x;
+    const float *v = reinterpret_cast<const float *>(s_xyz[1]) + 3u * threadIdx.x;
+    p.px[i] = x[0];
+    p.py[i] = x[1];
+    p.pz[i] = x[2];
+    p.vx[i] = vel ? v[0] : 0.0f;
+    p.vy[i] = vel ? v[1] : 0.0f;
+    p.vz[i] = vel ? v[2] : 0.0f;
+    p.id[i] = ids ? ids[k] : id_base + k;
+    if (ocell) ocell[i] = 0u;
+}
+
+// at[id] = the slot of each of the particles first .. first + n - 1. An id outside
+// 0 .. n - 1 raises *bad (host memory) instead.
+__global__ __launch_bounds__(256) void k_slots_by_id(const uint32_t *__restrict__ id, uint32_t first, uint32_t n,
+                                                     uint32_t *__restrict__ at, volatile uint32_t *bad)
 {
     const uint32_t k = blockIdx.x * 256u + threadIdx.x;
     if (k >= n) return;
-    const uint32_t i = first + k, id = p.id[i];
-    if (id >= n) {
-        atomicOr(bad, 1u);
-        return;
+    const uint32_t d = id[first + k];
+    if (d < n)
+        at[d] = first + k;
+    else
+        *bad = 1u;
+}
+
+// The particles first .. first + n - 1 by id as xyz triples (render/readback order, as
+// CGPUBaseParticleSimulator::integrate un-permutes by id,
+// src/CGPUBaseParticleSimulator.cpp:83-91). vel may be null. Nothing is written for an
+// id that no particle has (at[id] is then left from before or any word).
+//
+// Scattering the particles' words to host memory in slot order made a write over the
+// link of almost every 4-byte word: 292 us for 250,047 particles and 2.41 ms for
+// 1,048,576, against 117 us and 0.50 ms with the slots by id; 3.9 and 6.5 us for 1,620.
+__global__ __launch_bounds__(kTriples) void k_pack_by_id(ParticleSoA p, const uint32_t *__restrict__ at,
+                                                         uint32_t first, uint32_t n, float *__restrict__ pos,
+                                                         float *__restrict__ vel)
+{
+    __shared__ float4 s_xyz[2][kTriples * 3 / 4];
+    const uint32_t d0 = blockIdx.x * kTriples, d = d0 + threadIdx.x;
+    float *x = reinterpret_cast<float *>(s_xyz[0]) + 3u * threadIdx.x;
+    float *v = reinterpret_cast<float *>(s_xyz[1]) + 3u * threadIdx.x;
+    const uint32_t i = d < n ? at[d] : 0xFFFFFFFFu;
+    const bool found = i - first < n && p.id[i] == d;
+    if (found) {
+        x[0] = p.px[i];
+        x[1] = p.py[i];
+        x[2] = p.pz[i];
+        if (vel) {
+            v[0] = p.vx[i];
+            v[1] = p.vy[i];
+            v[2] = p.vz[i];
+        }
     }
-    pos[3 * (size_t) id + 0] = p.px[i];
-    pos[3 * (size_t) id + 1] = p.py[i];
-    pos[3 * (size_t) id + 2] = p.pz[i];
-    if (vel) {
-        vel[3 * (size_t) id + 0] = p.vx[i];
-        vel[3 * (size_t) id + 1] = p.vy[i];
-        vel[3 * (size_t) id + 2] = p.vz[i];
+    if (__syncthreads_and(found)) {
+        float4 *po = reinterpret_cast<float4 *>(pos + 3u * (size_t) d0);
+        float4 *vo = reinterpret_cast<float4 *>(vel + 3u * (size_t) d0);
+        for (uint32_t q = threadIdx.x; q < kTriples * 3 / 4; q += kTriples) po[q] = s_xyz[0][q];
+        if (!vel) return;
+        for (uint32_t q = threadIdx.x; q < kTriples * 3 / 4; q += kTriples) vo[q] = s_xyz[1][q];
+    } else if (found) {   // the last workgroup, and around an id that is missing
+        for (int c = 0; c < 3; ++c) {
+            pos[3u * (size_t) d + c] = x[c];
+            if (vel) vel[3u * (size_t) d + c] = v[c];
+        }
     }
 }
 
@@ -2262,11 +2332,20 @@ void launch_emit(const Emitter *em, uint32_t nem, Scene *scenes, const ParticleS
     hipLaunchKernelGGL(k_emit, dim3(nem), dim3(256), 0, st, em, scenes, p, key, cc, ocell, h);
 }
 
-void launch_scatter_by_id(const ParticleSoA &p, uint32_t first, uint32_t n, float *pos, float *vel, uint32_t *bad,
-                          hipStream_t st)
+void launch_unpack(const float *pos, const float *vel, const uint32_t *ids, uint32_t id_base, const ParticleSoA &p,
+                   uint32_t *ocell, uint32_t first, uint32_t n, hipStream_t st)
 {
     if (n == 0) return;
-    hipLaunchKernelGGL(k_scatter_by_id, dim3(blocks_for(n, 256)), dim3(256), 0, st, p, first, n, pos, vel, bad);
+    hipLaunchKernelGGL(k_unpack, dim3(blocks_for(n, kTriples)), dim3(kTriples), 0, st, (const float4 *) pos,
+                       (const float4 *) vel, ids, id_base, p, ocell, first, n);
+}
+
+void launch_pack_by_id(const ParticleSoA &p, uint32_t first, uint32_t n, uint32_t *at, float *pos, float *vel,
+                       uint32_t *bad, hipStream_t st)
+{
+    if (n == 0) return;
+    hipLaunchKernelGGL(k_slots_by_id, dim3(blocks_for(n, 256)), dim3(256), 0, st, p.id, first, n, at, bad);
+    hipLaunchKernelGGL(k_pack_by_id, dim3(blocks_for(n, kTriples)), dim3(kTriples), 0, st, p, at, first, n, pos, vel);
 }
 
 void launch_hash(const ParticleSoA &p, uint32_t *key, const CellCount &cc, const SceneTable &t, double h, hipStream_t st)
