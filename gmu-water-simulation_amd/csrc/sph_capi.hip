@@ -1364,11 +1364,11 @@ void sph_default_scene(sph_scene_desc *d, float box, uint32_t capacity)
 uint64_t sph_slot_bytes(uint32_t max_neighbours)
 {
     const uint64_t lists = max_neighbours == SPH_NEIGHBOUR_LISTS_OFF ? 0 : max_neighbours;
-    // pos/vel ping-pong 48, ids 8, keys and values 20, rho 4, records 40,
+    // pos/vel ping-pong 48, ids 8, keys and values 20, rho 4, records 32,
     // accelerations 12, counts 8, row masks (the default mode without
-    // lists), list entries, and 4 for the histograms, the group map and the
-    // scene's share of the cell table
-    return 48 + 8 + 20 + 4 + 4 * sph::kRecWords + 12 + 8 + (lists ? 4 * lists : 9 * 4 * sph::kMaskWords) + 4;
+    // lists), list entries, 4 for the readback's slots by id, and 8 for the
+    // histograms, the group map and the scene's share of the cell table and counts
+    return 48 + 8 + 20 + 4 + 4 * sph::kRecWords + 12 + 8 + (lists ? 4 * lists : 9 * 4 * sph::kMaskWords) + 4 + 8;
 }
 
 int sph_grid_res(float box)

@@ -1110,7 +1110,7 @@ constexpr uint32_t kBufWord3 = 0x00020000;  // descriptor word 3 of a gfx9 raw b
 // instruction) instead of 64-bit addresses, and reads outside the scene's
 // segment return 0 instead of faulting.
 struct BufView {
-    __amdgpu_buffer_rsrc_t px, py, pz, rho, rec;
+    __amdgpu_buffer_rsrc_t px, py, pz, rec;
 };
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void *base, uint32_t bytes)
@@ -1124,7 +1124,6 @@ __device__ __forceinline__ BufView buf_view(const ParticleSoA &p, const DensityF
     v.px = rsrc(p.px + s.poff, s.cap * 4u);
     v.py = rsrc(p.py + s.poff, s.cap * 4u);
     v.pz = rsrc(p.pz + s.poff, s.cap * 4u);
-    v.rho = rsrc(f.rho + s.poff, s.cap * 4u);
     v.rec = rsrc(f.rec + kRecWords * (size_t) s.poff, s.cap * (4u * kRecWords));
     return v;
 }
@@ -1347,19 +1346,10 @@ __device__ __forceinline__ float spiky_scale(double hr, float r2, const Consts &
 __device__ __forceinline__ void store_density(const DensityFields &f, const ParticleSoA &p, const Consts &k, uint32_t i,
                                               float density, float xi, float yi, float zi)
 {
-    const float pressure = k.gas_k * (density - k.rho0);
     f.rho[i] = density;
-    // rho*rho is exact in double, so this is p / pow(rho, 2)
-    const double prr = (double) pressure / ((double) density * (double) density);
-    const double rinv = 1.0 / (double) density;
-    // the record, as five 8-byte stores (records are 8-byte aligned)
-    uint2 *rec = reinterpret_cast<uint2 *>(f.rec + kRecWords * (size_t) i);
-    const uint64_t pb = __builtin_bit_cast(uint64_t, prr), rb = __builtin_bit_cast(uint64_t, rinv);
-    rec[0] = make_uint2(__float_as_uint(xi), __float_as_uint(yi));
-    rec[1] = make_uint2(__float_as_uint(zi), __float_as_uint(p.vx[i]));
-    rec[2] = make_uint2(__float_as_uint(p.vy[i]), __float_as_uint(p.vz[i]));
-    rec[3] = make_uint2((uint32_t) pb, (uint32_t) (pb >> 32));
-    rec[4] = make_uint2((uint32_t) rb, (uint32_t) (rb >> 32));
+    float4 *rec = reinterpret_cast<float4 *>(f.rec + kRecWords * (size_t) i);
+    rec[0] = make_float4(xi, yi, zi, p.vx[i]);
+    rec[1] = make_float4(p.vy[i], p.vz[i], density, k.gas_k * (density - k.rho0));
 }
 
 // updateDensityPressure, src/CCPUParticleSimulator.cpp:93-141. Also stores
@@ -1438,34 +1428,45 @@ struct ForceSums {
 // The neighbour data one force pair reads, loaded one pair ahead of its use so
 // that the loads of pair q+1 are in flight while pair q is computed.
 struct PairData {
-    uint32_t off;   // byte offset of the neighbour's record: 40 * its slot
-    float x, y, z, vx, vy, vz;
-    double prr, rinv;
+    uint32_t off;   // byte offset of the neighbour's record: 32 * its slot
+    float x, y, z, vx, vy, vz, rho, p;
 };
+
+// What the pair terms divide by: 1/rho to within 2^-52, and p/rho^2 rounded as the
+// division rounds it.
+//
+// 1/rho takes the single-precision estimate (within 2^-22) through one step of third
+// order, its error cubed: below 2^-66 and the two roundings. The quotient is p times
+// its square, then corrected by the remainder, which is exact by FMA (rho^2 is exact,
+// of 48 bits, and the quotient within 3 units of its last place). The corrected sum is
+// within 2^-50 units of p/rho^2 before it is rounded, and no p/rho^2 of two floats
+// lies within 2^-49 units of the middle between two doubles: so it rounds the same
+// way. rho is a normal float wherever a neighbour is accepted (a particle's own term
+// is in its sum).
+__device__ __forceinline__ void density_quotients(float rho, float p, double &rinv, double &prr)
+{
+    const double d = (double) rho, y = (double) __builtin_amdgcn_rcpf(rho);
+    const double e = __builtin_fma(-d, y, 1.0);
+    rinv = __builtin_fma(y, __builtin_fma(e, e, e), y);
+    const double d2 = d * d, y2 = rinv * rinv, pd = (double) p;
+    const double q = pd * y2;
+    prr = __builtin_fma(__builtin_fma(-d2, q, pd), y2, q);
+}
 
 // p/rho^2 of slot i from its record.
 __device__ __forceinline__ double own_prr(const DensityFields &f, uint32_t i)
 {
-    const uint2 w = *reinterpret_cast<const uint2 *>(f.rec + kRecWords * (size_t) i + 6);
-    return __builtin_bit_cast(double, (uint64_t) w.x | ((uint64_t) w.y << 32));
+    const float2 w = *reinterpret_cast<const float2 *>(f.rec + kRecWords * (size_t) i + 6);
+    double rinv, prr;
+    density_quotients(w.x, w.y, rinv, prr);
+    return prr;
 }
 
-// The record at byte offset o (40 * slot).
+// The record at byte offset o (32 * slot).
 __device__ __forceinline__ PairData load_pair_at(const BufView &bv, uint32_t o)
 {
     const float4 a = ld4(bv.rec, o), b = ld4(bv.rec, o + 16u);
-    const uint2 c = ld2u(bv.rec, o + 32u);
-    PairData d;
-    d.off = o;
-    d.x = a.x;
-    d.y = a.y;
-    d.z = a.z;
-    d.vx = a.w;
-    d.vy = b.x;
-    d.vz = b.y;
-    d.prr = __builtin_bit_cast(double, (uint64_t) __float_as_uint(b.z) | ((uint64_t) __float_as_uint(b.w) << 32));
-    d.rinv = __builtin_bit_cast(double, (uint64_t) c.x | ((uint64_t) c.y << 32));
-    return d;
+    return PairData{o, a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 }
 
 __device__ __forceinline__ PairData load_pair(const BufView &bv, uint32_t j)
@@ -1493,15 +1494,47 @@ __device__ __forceinline__ PairTerms pair_terms(const BufView &bv, const Consts 
     const float sg = spiky_scale(hr, r2, k);
     float gx, gy, gz;
     div3_small_divisor(dx * sg, dyv * sg, dzv * sg, (float) r, gx, gy, gz, y2);
-    const float pf = (float) (ai + n.prr);
+    double rinv, prr;
+    density_quotients(n.rho, n.p, rinv, prr);
+    const float pf = (float) (ai + prr);
     PairTerms t;
     t.px = gx * pf;
     t.py = gy * pf;
     t.pz = gz * pf;
     const float lap = (float) (k.visc * hr);
-    div3_rcp((n.vx - vxi) * lap, (n.vy - vyi) * lap, (n.vz - vzi) * lap, n.rinv,
-             [&]() { return ldf(bv.rho, n.off / 10u); }, t.vx, t.vy, t.vz);
+    div3_rcp((n.vx - vxi) * lap, (n.vy - vyi) * lap, (n.vz - vzi) * lap, rinv, [&]() { return n.rho; }, t.vx, t.vy,
+             t.vz);
     return t;
+}
+
+// pair_terms without its branches, for two pairs side by side: a wave's FP64 operations
+// depend on each other, and those of one pair fill the waits of the other's. Returns
+// whether the terms must be redone (redo_terms): the spiky factor lies near a float
+// boundary, or a quotient is not a normal float.
+__device__ __forceinline__ bool try_terms(const Consts &k, const PairData &n, float xi, float yi, float zi, float vxi,
+                                          float vyi, float vzi, double ai, PairTerms &t)
+{
+    const float dx = xi - n.x, dyv = yi - n.y, dzv = zi - n.z;
+    const float r2 = dx * dx + dyv * dyv + dzv * dzv;
+    const double x2 = (double) r2, y2 = __builtin_amdgcn_rsq(x2);
+    const double r = sqrt_with_rsq(x2, y2);
+    const double hr = k.h - r, sgd = k.spiky * (hr * hr);
+    const float sg = (float) sgd;
+    const double rb = rcp_from((double) (float) r, y2);
+    const float gx = (float) ((double) (dx * sg) * rb), gy = (float) ((double) (dyv * sg) * rb),
+                gz = (float) ((double) (dzv * sg) * rb);
+    double rinv, prr;
+    density_quotients(n.rho, n.p, rinv, prr);
+    const float pf = (float) (ai + prr);
+    t.px = gx * pf;
+    t.py = gy * pf;
+    t.pz = gz * pf;
+    const float lap = (float) (k.visc * hr);
+    t.vx = (float) ((double) ((n.vx - vxi) * lap) * rinv);
+    t.vy = (float) ((double) ((n.vy - vyi) * lap) * rinv);
+    t.vz = (float) ((double) ((n.vz - vzi) * lap) * rinv);
+    // (bitwise operators: no branch)
+    return (int) near_float_boundary(sgd) | (int) !all_normal3(gx, gy, gz) | (int) !all_normal3(t.vx, t.vy, t.vz);
 }
 
 __device__ __forceinline__ void add_terms(ForceSums &a, const PairTerms &t)
@@ -1643,40 +1676,66 @@ __device__ __forceinline__ ForceSums mask_sums(const BufView &bv, const uint32_t
     return a;
 }
 
-// Drains a lane's queue of mask words (nq entries of two 32-bit words at
-// stride T: the bits and the record offset of bit 0, 40 * its slot) into its
-// force sums: the set bits of each word in ascending order, word after word. Two
-// pairs are in flight, as in drain_pairs; a lane with no pair left loads the
-// record at `fallback` (an offset) and adds nothing. A bit's record offset is
-// the word's plus a 24-bit product, so no full 32-bit multiply per pair.
+// The largest value of the wave's active lanes, below 1024.
+__device__ __forceinline__ uint32_t wave_max(uint32_t v)
+{
+    uint32_t top = 0;
+    bool most = true;   // the lane's bits so far are the largest value's
+#pragma unroll
+    for (int b = 9; b >= 0; --b) {
+        const bool set = most && (v >> b & 1u);
+        if (__any(set)) {
+            top |= 1u << b;
+            most = set;
+        }
+    }
+    return top;
+}
+
+// Drains a lane's queue of mask words (entries of two 32-bit words at stride T: the
+// bits, `pairs` in all, and the record offset of bit 0, 32 * its slot) into its force
+// sums: the set bits of each word in ascending order, word after word. Two pairs are
+// computed side by side while the records of the next two and the word after the one
+// at hand are on their way; a lane with no pair left loads the record at `fallback` (an
+// offset) and adds nothing. The trips are counted for the wave: around a loop that
+// each lane leaves by itself the compiler copies the sums on every trip. The entry
+// behind the last one may be read.
 template <int T>
-__device__ __forceinline__ void drain_words(const BufView &bv, const Consts &k, const uint32_t *qw, int nq,
+__device__ __forceinline__ void drain_words(const BufView &bv, const Consts &k, const uint32_t *qw, uint32_t pairs,
                                             uint32_t fallback, float xi, float yi, float zi, float vxi, float vyi,
                                             float vzi, double ai, ForceSums &a)
 {
-    int q = 0;
-    uint32_t m = 0, o0 = 0;
-    auto next = [&](uint32_t &o) {
-        if (m == 0u && q < nq) {
-            m = qw[(2 * q) * T];
-            o0 = qw[(2 * q + 1) * T];
-            ++q;
+    const uint32_t trips = wave_max(pairs);
+    uint32_t m = qw[0], o0 = qw[T], m1 = qw[2 * T], o1 = qw[3 * T];
+    auto next = [&](uint32_t e) {   // the record of pair e
+        if (e >= pairs) return fallback;
+        if (m == 0u) {
+            m = m1;
+            o0 = o1;
+            qw += 2 * T;
+            m1 = qw[2 * T];
+            o1 = qw[3 * T];
         }
-        const bool ok = m != 0u;
-        o = ok ? o0 + __umul24((uint32_t) __builtin_ctz(m), 4u * kRecWords) : fallback;
+        const uint32_t o = o0 + (uint32_t) __builtin_ctz(m) * (4u * kRecWords);
         m &= m - 1u;
-        return ok;
+        return o;
     };
-    uint32_t oa, ob;
-    bool va = next(oa);
-    PairData pa = load_pair_at(bv, oa);
-    while (__any(va)) {
-        const bool vb = next(ob);
-        const PairData pb = load_pair_at(bv, ob);
-        if (va) force_pair(bv, k, pa, xi, yi, zi, vxi, vyi, vzi, ai, a);
-        va = next(oa);
-        pa = load_pair_at(bv, oa);
-        if (vb) force_pair(bv, k, pb, xi, yi, zi, vxi, vyi, vzi, ai, a);
+    const uint32_t oa = next(0), ob = next(1);
+    PairData na = load_pair_at(bv, oa), nb = load_pair_at(bv, ob);
+    for (uint32_t e = 0; e < trips; e += 2) {
+        const PairData pa = na, pb = nb;
+        const uint32_t oc = next(e + 2), od = next(e + 3);
+        na = load_pair_at(bv, oc);
+        nb = load_pair_at(bv, od);
+        PairTerms ta, tb;
+        const bool ra = try_terms(k, pa, xi, yi, zi, vxi, vyi, vzi, ai, ta);
+        const bool rb = try_terms(k, pb, xi, yi, zi, vxi, vyi, vzi, ai, tb);
+        if (__builtin_expect((int) ra | (int) rb, 0)) {
+            ta = pair_terms(bv, k, pa, xi, yi, zi, vxi, vyi, vzi, ai);
+            tb = pair_terms(bv, k, pb, xi, yi, zi, vxi, vyi, vzi, ai);
+        }
+        if (e < pairs) add_terms(a, ta);
+        if (e + 1 < pairs) add_terms(a, tb);
     }
 }
 
@@ -1686,9 +1745,16 @@ constexpr unsigned kWaitVmcnt0 = 0x0F70;
 // The force sums of particle i from the row masks, as mask_sums, with another
 // division of the work: the wave reads the rows and words together (coalesced)
 // and each lane queues its non-empty words, without its own bit, in LDS (`qw`,
-// W entries at stride T); drain_words runs through every lane's queue when one
-// is full and at the end. With W large enough for a particle's words there is
-// one drain per wave and no per-bit fill rounds, at the price of more LDS.
+// W entries at stride T, and room for another); drain_words runs through every lane's
+// queue when one is full and at the end. With W large enough for a particle's words
+// there is one drain per wave and no per-bit fill rounds, at the price of more LDS.
+//
+// Bound by vector instructions for four fifths of its time and by the last waves to
+// end for the rest (a wave takes 50 us on average, 80 to 100 us at most, with three or
+// four on a SIMD). The force pass of 50,653 / 300,007 / 1,048,576 particles and of 128
+// scenes with 2.3 million takes 37.1 / 108.6 / 331 / 419 us; with 40-byte records and
+// one pair after the other 38.7 / 113.7 / 353 / 454 us, bound by the L1's accesses, and
+// with 32-byte records alone 40.4 / 114.8 / 352 / 438 us.
 template <bool kRef, int T, int W>
 __device__ __forceinline__ ForceSums mask_sums_queue(const BufView &bv, const uint32_t *__restrict__ cell,
                                                      const uint32_t *__restrict__ start,
@@ -1706,12 +1772,23 @@ __device__ __forceinline__ ForceSums mask_sums_queue(const BufView &bv, const ui
     uint32_t m0[9];
 #pragma unroll
     for (int r = 0; r < 9; ++r) m0[r] = masks[mask_word(i, r, 0)];
-    int nq = 0;
-    for (int r = 0; r < 9; ++r) {
-        uint32_t jrun, jend;
-        row_run<kRef>(rb, s, start, x, y, z, r, jrun, jend);
-        const uint32_t nw = (jend - jrun + kMaskWordBits - 1) / kMaskWordBits;
-        for (uint32_t w = 0; __any(w < nw); ++w) {
+    int r = -1;
+    uint32_t w = 0, nw = 0, jrun = 0;   // the lane's words of row r, the next one and the row's first candidate
+    bool more = true;
+    do {
+        uint32_t nq = 0, pairs = 0;
+        do {
+            if (!__any(w < nw)) {
+                if (++r == 9) {
+                    more = false;
+                    break;
+                }
+                uint32_t jend;
+                row_run<kRef>(rb, s, start, x, y, z, r, jrun, jend);
+                nw = (jend - jrun + kMaskWordBits - 1) / kMaskWordBits;
+                w = 0;
+                continue;
+            }
             uint32_t m = w >= nw ? 0u : w == 0 ? m0[r] : masks[mask_word(i, r, w)];
             const uint32_t j0 = jrun + kMaskWordBits * w, self = li - j0;
             if (self < kMaskWordBits) m &= ~(1u << self);
@@ -1720,14 +1797,12 @@ __device__ __forceinline__ ForceSums mask_sums_queue(const BufView &bv, const ui
                 qw[(2 * nq + 1) * T] = j0 * (4u * kRecWords);
                 ++nq;
             }
-            if (__any(nq == W)) {
-                drain_words<T>(bv, k, qw, nq, fallback, xi, yi, zi, vxi, vyi, vzi, ai, a);
-                __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);   // the drain's last, unused loads
-                nq = 0;
-            }
-        }
-    }
-    drain_words<T>(bv, k, qw, nq, fallback, xi, yi, zi, vxi, vyi, vzi, ai, a);
+            pairs += (uint32_t) __popc(m);
+            ++w;
+        } while (!__any(nq == (uint32_t) W));
+        drain_words<T>(bv, k, qw, pairs, fallback, xi, yi, zi, vxi, vyi, vzi, ai, a);
+        __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);   // the drain's last, unused loads
+    } while (more);
     return a;
 }
 
@@ -1744,10 +1819,13 @@ __device__ __forceinline__ void accel_from_sums(const ForceSums &a, float rhoi, 
     az = ((fpz + fvz) + fgz) / rhoi;
 }
 
+constexpr int kPhaseWords = 24;   // queued mask words of the phase's force pass
+
 // The acceleration of particle i. Neighbours come from the density pass's list
-// when one was kept (each lane running through its own list); otherwise (or on
-// overflow) the cells are walked again in the same order.
-template <bool kRef, int T, int U>
+// when one was kept (each lane running through its own list), with kPhaseQueue from
+// its row masks; otherwise (or on overflow) the cells are walked again in the same
+// order.
+template <bool kRef, int T, int U, bool kPhaseQueue = false>
 __device__ __forceinline__ void sph_accel(const ParticleSoA &p, const uint32_t *__restrict__ cell,
                                           const uint32_t *__restrict__ start, const DensityFields &f,
                                           const NeighbourList &nl, uint32_t *my, uint32_t i, uint32_t li,
@@ -1771,10 +1849,15 @@ __device__ __forceinline__ void sph_accel(const ParticleSoA &p, const uint32_t *
             }
             force_pair(bv, k, cur, xi, yi, zi, vxi, vyi, vzi, ai, a);
         }
-    } else if (nl.mode == kNbMasks && nl.cnt[i] == 0) {
-        a = mask_sums<kRef, T, kListCap, 0>(bv, cell, start, nl.masks, my, i, li, s, k, xi, yi, zi, vxi, vyi, vzi, ai);
     } else {
-        a = walk_sums<kRef, T, U>(bv, cell, start, my, i, li, s, k, xi, yi, zi, vxi, vyi, vzi, ai);
+        bool walk = true;
+        if constexpr (kPhaseQueue) {
+            walk = nl.cnt[i] != 0;
+            if (!walk)
+                a = mask_sums_queue<kRef, T, kPhaseWords>(bv, cell, start, nl.masks, my, i, li, s, k, xi, yi, zi, vxi,
+                                                          vyi, vzi, ai);
+        }
+        if (walk) a = walk_sums<kRef, T, U>(bv, cell, start, my, i, li, s, k, xi, yi, zi, vxi, vyi, vzi, ai);
     }
     accel_from_sums(a, rhoi, s, k, ax, ay, az);
 }
@@ -1873,24 +1956,33 @@ __device__ __forceinline__ void integrate_one(float xi, float yi, float zi, floa
     nvz = (nz - zi) / dt;
 }
 
-constexpr int kPhaseThreads = 256;   // workgroup of the phase-by-phase kernels
 constexpr int kPhaseUnroll = 4;
 
-template <bool kRef>
-__global__ __launch_bounds__(kPhaseThreads) void k_forces(ParticleSoA p, const uint32_t *__restrict__ cell,
-                                                          const uint32_t *__restrict__ start, DensityFields f,
-                                                          NeighbourList nl, float *__restrict__ ax,
-                                                          float *__restrict__ ay, float *__restrict__ az,
-                                                          SceneTable t, Consts k)
+// Workgroup of the phase's force pass: one wave with row masks, as the fused pass has.
+// With lists of pairs filled bit by bit (mask_sums) it took 152 us for 250,047
+// particles, with the word queue 83.
+template <bool kMasks>
+constexpr int phase_threads()
 {
-    __shared__ uint32_t lst[kListCap * kPhaseThreads];
-    const uint32_t first = xcd_block(blockIdx.x, gridDim.x) * (uint32_t) kPhaseThreads, i = first + threadIdx.x;
+    return kMasks ? 64 : 256;
+}
+
+template <bool kRef, bool kMasks>
+__global__ __launch_bounds__(phase_threads<kMasks>()) void k_forces(ParticleSoA p, const uint32_t *__restrict__ cell,
+                                                                    const uint32_t *__restrict__ start,
+                                                                    DensityFields f, NeighbourList nl,
+                                                                    float *__restrict__ ax, float *__restrict__ ay,
+                                                                    float *__restrict__ az, SceneTable t, Consts k)
+{
+    constexpr int T = phase_threads<kMasks>();
+    __shared__ uint32_t lst[(kMasks ? 2 * kPhaseWords + 2 : kListCap) * T];
+    const uint32_t first = xcd_block(blockIdx.x, gridDim.x) * (uint32_t) T, i = first + threadIdx.x;
     const Scene s = block_scene(t, first);
     const uint32_t li = i - s.poff;
     if (i >= t.nslots || li >= s.n) return;
     float a0, a1, a2;
-    sph_accel<kRef, kPhaseThreads, kPhaseUnroll>(p, cell, start, f, nl, lst + threadIdx.x, i, li, s, k, p.px[i], p.py[i],
-                                           p.pz[i], p.vx[i], p.vy[i], p.vz[i], a0, a1, a2);
+    sph_accel<kRef, T, kPhaseUnroll, kMasks>(p, cell, start, f, nl, lst + threadIdx.x, i, li, s, k, p.px[i], p.py[i],
+                                             p.pz[i], p.vx[i], p.vy[i], p.vz[i], a0, a1, a2);
     ax[i] = a0;
     ay[i] = a1;
     az[i] = a2;
@@ -1947,7 +2039,8 @@ __global__ __launch_bounds__(T) void k_forces_fused(ParticleSoA p, const uint32_
 {
     static_assert(kGroupSlots % T == 0, "a workgroup must lie in one slot group");
     constexpr bool kLists = kMode == kNbLists;
-    __shared__ uint32_t lst[(kMode == kNbMasks && C > kListCap ? C : kListCap) * T];
+    constexpr int kLst = kMode != kNbMasks ? 0 : kQueue ? C + 2 : C;
+    __shared__ uint32_t lst[(kLst > kListCap ? kLst : kListCap) * T];
     __shared__ float4 s_owner[kLists ? 2 * T : 1];
     __shared__ float4 s_acc[kLists ? 2 * T : 1];
     __shared__ uint16_t s_items[kLists ? kLevelWindow * T : 1];
@@ -2549,12 +2642,15 @@ void launch_forces(const ParticleSoA &p, const uint32_t *cell, const uint32_t *s
                                    k, ref, st);
         return;
     }
-    if (ref)
-        hipLaunchKernelGGL(k_forces<true>, dim3(blocks_for(t.nslots, kPhaseThreads)), dim3(kPhaseThreads), 0, st, p,
-                           cell, start, f, nl, ax, ay, az, t, k);
-    else
-        hipLaunchKernelGGL(k_forces<false>, dim3(blocks_for(t.nslots, kPhaseThreads)), dim3(kPhaseThreads), 0, st, p,
-                           cell, start, f, nl, ax, ay, az, t, k);
+#define SPH_PHASE(ref_, masks_)                                                                        \
+    hipLaunchKernelGGL((k_forces<ref_, masks_>), dim3(blocks_for(t.nslots, phase_threads<masks_>())),   \
+                       dim3(phase_threads<masks_>()), 0, st, p, cell, start, f, nl, ax, ay, az, t, k)
+    if (nl.mode == kNbMasks) {
+        if (ref) SPH_PHASE(true, true); else SPH_PHASE(false, true);
+    } else {
+        if (ref) SPH_PHASE(true, false); else SPH_PHASE(false, false);
+    }
+#undef SPH_PHASE
 }
 
 void launch_collide(const ParticleSoA &p, float *ax, float *ay, float *az, const SceneTable &t, const Consts &k,

@@ -159,7 +159,7 @@ sph_status sph_step(sph_ctx *ctx, uint32_t nsteps, float *ms_out);
  * calls that overlap on one GPU (other threads or streams) race and must not be made. */
 #define SPH_NOALLOC_MAX_PARTICLES 65536u
 #define SPH_NOALLOC_MAX_CELLS 262144u
-#define SPH_NOALLOC_SCRATCH_BYTES 46138880u
+#define SPH_NOALLOC_SCRATCH_BYTES 45614592u
 typedef struct {
     float *px, *py, *pz;
     float *vx, *vy, *vz;
@@ -318,7 +318,8 @@ sph_status sph_set_graphs(sph_ctx *ctx, int enable);
  *   SPH_NEIGHBOURS_LISTS reads neighbour lists the density pass kept (only if the context
  *                        was created with max_neighbours > 0);
  *   SPH_NEIGHBOURS_MASKS reads per-row masks of the accepted candidates the density pass
- *                        kept (576 bytes per slot).
+ *                        kept (576 bytes per slot); up to 40,960 slots in use, 16-bit
+ *                        neighbour slots kept there, four lanes to a particle.
  * A new context uses variant 12 and SPH_NEIGHBOURS_MASKS, or SPH_NEIGHBOURS_LISTS when it
  * was created with max_neighbours > 0. Results are identical for every choice. */
 #define SPH_NUM_VARIANTS 21
