@@ -980,9 +980,9 @@ sph_status ensure_upload(sph_ctx *c, uint32_t n)
     const uint32_t want = round_up(std::min(n, kUploadPart), 256);
     if (want <= c->up_cap) return SPH_OK;
     free_upload(c);
-    for (int part = 0; part < 2; ++part) {
+    for (int part = 0; part < (want < kUploadPart ? 1 : 2); ++part) {   // a small one is never refilled
         SPH_HIP(hipHostMalloc((void **) &c->up[part], (size_t) want * 28, hipHostMallocDefault));
-        SPH_HIP(hipEventCreateWithFlags(&c->up_read[part], hipEventDisableTiming));
+        if (want == kUploadPart) SPH_HIP(hipEventCreateWithFlags(&c->up_read[part], hipEventDisableTiming));
     }
     c->up_cap = want;
     return SPH_OK;
@@ -1009,7 +1009,7 @@ sph_status write_slots(sph_ctx *c, const float *pos3, const float *vel3, const u
         sph::launch_unpack(pos, vel3 ? vel : nullptr, ids ? id : nullptr, id_base + k, c->soa(c->cur, c->id_cur),
                            c->ref_order() ? c->ocell : nullptr, first + k, m, c->stream);
         st = launch_error("upload launch");
-        if (!st) SPH_HIP(hipEventRecord(c->up_read[part], c->stream));
+        if (!st && n > c->up_cap) SPH_HIP(hipEventRecord(c->up_read[part], c->stream));
     }
     SPH_HIP(hipStreamSynchronize(c->stream));
     return st;
