@@ -49,7 +49,7 @@ sph_status fail(sph_status code, const std::string &msg)
     } while (0)
 
 constexpr int kProfileSlots = 256;          // event pairs buffered before a forced drain
-constexpr uint32_t kMaxSceneSlots = 1u << 26;  // 40-byte records of a scene stay below 4 GiB (buffer offsets)
+constexpr uint32_t kMaxSceneSlots = 1u << 26;  // 32-byte records of a scene stay below 4 GiB (buffer offsets)
 constexpr uint32_t kMaxPool = 1u << 31;
 constexpr uint32_t kNoScene = 0xFFFFFFFFu;
 
