@@ -2105,7 +2105,7 @@ __global__ __launch_bounds__(T) void k_forces_fused(ParticleSoA p, const uint32_
 // one wave or none, and takes as long as its longest wave, a wave alone issuing a vector
 // instruction every 7 cycles or so. Here four lanes share a particle, 16 particles a
 // wave, and the particle's terms are still added in the canonical order: at 4,096
-// particles 25.9 -> 17.4 us for the density and 19.2 -> 9.2 us for the force pass, at
+// particles 25.9 -> 19.3 us for the density and 19.2 -> 8.3 us for the force pass, at
 // 50,653 no longer (51 -> 77 and 39 -> 23 us), and at 1,048,576 the shared force pass
 // has half as much again of vector instructions (357 -> 486 us).
 
@@ -2276,8 +2276,7 @@ __global__ __launch_bounds__(64) void k_forces_split(ParticleSoA p, const uint32
         // loaded by lanes without a pair, never added (a record offset)
         const uint32_t fallback = (li + 1 < s.n ? li + 1 : li - 1) * (4u * kRecWords);
         auto offset = [&](uint32_t e) { return e < cnt_i ? (uint32_t) nb[e * 64u] * (4u * kRecWords) : fallback; };
-        auto add = [&](const PairData &n, bool have) {
-            PairTerms v = pair_terms(bv, k, n, xi, yi, zi, vxi, vyi, vzi, ai);
+        auto add = [&](PairTerms v, bool have) {
             if (!have) v = PairTerms{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
 #define SPH_QUAD_ADD(c) \
     a.c = a.c + quad_lane<0>(v.c); \
@@ -2299,8 +2298,16 @@ __global__ __launch_bounds__(64) void k_forces_split(ParticleSoA p, const uint32
             const PairData pc = load_pair_at(bv, oc), pd = load_pair_at(bv, od);
             oc = offset(e + 16u);
             od = offset(e + 20u);
-            add(pa, e < cnt_i);
-            add(pb, e + 4u < cnt_i);
+            const bool ha = e < cnt_i, hb = e + 4u < cnt_i;
+            PairTerms ta, tb;
+            const bool ra = try_terms(k, pa, xi, yi, zi, vxi, vyi, vzi, ai, ta);
+            const bool rb = try_terms(k, pb, xi, yi, zi, vxi, vyi, vzi, ai, tb);
+            if (__builtin_expect((int) ra | (int) rb, 0)) {
+                ta = pair_terms(bv, k, pa, xi, yi, zi, vxi, vyi, vzi, ai);
+                tb = pair_terms(bv, k, pb, xi, yi, zi, vxi, vyi, vzi, ai);
+            }
+            add(ta, ha);
+            add(tb, hb);
             pa = pc;
             pb = pd;
         }
