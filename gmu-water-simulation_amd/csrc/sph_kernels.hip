@@ -1676,13 +1676,14 @@ __device__ __forceinline__ ForceSums mask_sums(const BufView &bv, const uint32_t
     return a;
 }
 
-// The largest value of the wave's active lanes, below 1024.
+// The largest value of the wave's active lanes; the values are at most kMost.
+template <uint32_t kMost>
 __device__ __forceinline__ uint32_t wave_max(uint32_t v)
 {
     uint32_t top = 0;
     bool most = true;   // the lane's bits so far are the largest value's
 #pragma unroll
-    for (int b = 9; b >= 0; --b) {
+    for (int b = 31 - __builtin_clz(kMost); b >= 0; --b) {
         const bool set = most && (v >> b & 1u);
         if (__any(set)) {
             top |= 1u << b;
@@ -1699,13 +1700,13 @@ __device__ __forceinline__ uint32_t wave_max(uint32_t v)
 // at hand are on their way; a lane with no pair left loads the record at `fallback` (an
 // offset) and adds nothing. The trips are counted for the wave: around a loop that
 // each lane leaves by itself the compiler copies the sums on every trip. The entry
-// behind the last one may be read.
-template <int T>
+// behind the last one may be read. Up to W entries, so up to 32 W pairs.
+template <int T, int W>
 __device__ __forceinline__ void drain_words(const BufView &bv, const Consts &k, const uint32_t *qw, uint32_t pairs,
                                             uint32_t fallback, float xi, float yi, float zi, float vxi, float vyi,
                                             float vzi, double ai, ForceSums &a)
 {
-    const uint32_t trips = wave_max(pairs);
+    const uint32_t trips = wave_max<kMaskWordBits * W>(pairs);
     uint32_t m = qw[0], o0 = qw[T], m1 = qw[2 * T], o1 = qw[3 * T];
     auto next = [&](uint32_t e) {   // the record of pair e
         if (e >= pairs) return fallback;
@@ -1800,7 +1801,7 @@ __device__ __forceinline__ ForceSums mask_sums_queue(const BufView &bv, const ui
             pairs += (uint32_t) __popc(m);
             ++w;
         } while (!__any(nq == (uint32_t) W));
-        drain_words<T>(bv, k, qw, pairs, fallback, xi, yi, zi, vxi, vyi, vzi, ai, a);
+        drain_words<T, W>(bv, k, qw, pairs, fallback, xi, yi, zi, vxi, vyi, vzi, ai, a);
         __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);   // the drain's last, unused loads
     } while (more);
     return a;
