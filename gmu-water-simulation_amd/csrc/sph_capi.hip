@@ -754,7 +754,7 @@ sph_status run_grid_reference(sph_ctx *c)
         radix_sort(c, c->gold, nullptr, c->tiles_d, (uint32_t) c->tiles_h.size(), c->sort_bits);
         sph::launch_cell_start(c->key_s, n, C, c->cstart, c->stream);
         sph::launch_ref_counts(c->ref, c->gold, c->key_h, n, C, c->stream);
-        sph::launch_ref_bucket(c->ref, C, c->cstart, c->val_s, c->key_h, c->stream);
+        sph::launch_ref_bucket(c->ref, n, C, c->cstart, c->val_s, c->key_h, c->stream);
         sph::launch_ref_movers(c->ref, c->gold, c->key_h, n, C, c->stream);
         radix_sort(c, c->ref.mkey, c->ref.mval, c->tiles_flat_d, (uint32_t) c->tiles_flat_h.size(), c->flat_bits);
     }

@@ -197,7 +197,7 @@ struct RefBuffers {
 void launch_ref_prepare(const uint32_t *ocell, uint32_t *gold, const SceneTable &t, hipStream_t st);
 void launch_ref_counts(const RefBuffers &r, const uint32_t *gold, const uint32_t *gnew, uint32_t n, uint32_t ncells,
                        hipStream_t st);
-void launch_ref_bucket(const RefBuffers &r, uint32_t ncells, const uint32_t *ostart, const uint32_t *perm,
+void launch_ref_bucket(const RefBuffers &r, uint32_t n, uint32_t ncells, const uint32_t *ostart, const uint32_t *perm,
                        const uint32_t *gnew, hipStream_t st);
 void launch_ref_movers(const RefBuffers &r, const uint32_t *gold, const uint32_t *gnew, uint32_t n, uint32_t ncells,
                        hipStream_t st);

@@ -885,134 +885,196 @@ __global__ __launch_bounds__(256) void k_ref_count(const uint32_t *__restrict__ 
 // that filled hole h - 1; a mover at position q > K has rank L - q; one at K follows
 // the last hole as if it were the next.
 //
-// A wave takes a cell, its workgroup together a cell of more than 64 entries. One
-// thread a cell followed every bucket entry by entry: 6.3 ms for the 16,000 particles
-// that are all in cell 0 before a scene's first step, which now take 60 us, bound by the
-// dependent reads of 16 rounds; 4.5 us in the steps after it.
+// Grids of up to kBucketWaveCells cells: a wave takes a cell, its workgroup together a
+// cell of more than 64 entries (k_ref_bucket). One thread a cell followed every bucket
+// entry by entry: 6.3 ms for the 16,000 particles that are all in cell 0 before a
+// scene's first step, which now take 60 us, bound by the dependent reads of 16 rounds;
+// 4.5 us in the steps after it.
+//
+// Larger grids: most cells are empty or hold a few particles, so a lane takes a cell of
+// up to kLaneBucket entries (k_ref_bucket_lanes), bound by reading the tables, and lists
+// the others for k_ref_bucket, whose workgroups go through the list. Grid phases by
+// lanes and by waves, us: 24^3 cells with 1,728 particles 99.5 / 98.5, with 27,648
+// 114.9 / 109.3; 28^3 with 2,744 103.1 / 105.1, with 43,904 121.7 / 117.2; 32^3 with
+// 4,096 114.3 / 118.8, with 65,536 129.7 / 129.2; 44^3 with 42,592 154.5 / 174.2;
+// 100^3 with 125,000 523 / 800. (A launch of a wave a cell also ends at 2^32 / 64 cells.)
 constexpr uint32_t kBucketBlock = 4;   // cells (waves) a workgroup
+constexpr uint32_t kBucketWaveCells = 16384;
+constexpr uint32_t kLaneBucket = 32;   // the bits of a word
 
-__global__ __launch_bounds__(64 * kBucketBlock) void k_ref_bucket(uint32_t ncells, const uint32_t *__restrict__ ostart,
+// The cells of up to kLaneBucket entries; the others go to `list`, their number to
+// nstay[ncells] (zero before the call, as the other words of nstay).
+__global__ __launch_bounds__(256) void k_ref_bucket_lanes(uint32_t ncells, const uint32_t *__restrict__ ostart,
+                                                          const uint32_t *__restrict__ perm,
+                                                          const uint32_t *__restrict__ gnew,
+                                                          const uint32_t *__restrict__ eoff,
+                                                          uint32_t *__restrict__ list, uint32_t *__restrict__ rk,
+                                                          uint32_t *__restrict__ epos, uint32_t *__restrict__ nstay)
+{
+    const uint32_t c = blockIdx.x * 256u + threadIdx.x;
+    if (c >= ncells) return;
+    const uint32_t a = ostart[c], n = ostart[c + 1] - a;
+    const uint32_t e0 = eoff[c], len = n + (eoff[c + 1] - e0);
+    if (len == 0u) return;
+    if (len > kLaneBucket) {
+        list[atomicAdd(&nstay[ncells], 1u)] = c;
+        return;
+    }
+    uint32_t m = len > n ? (~0u >> (32u - (len - n))) << n : 0u;   // bit q: entry q stays
+#pragma unroll 4
+    for (uint32_t q = 0; q < n; ++q) m |= (uint32_t) (gnew[perm[a + q]] == c) << q;
+    const uint32_t stays = (uint32_t) __popc(m);
+    nstay[c] = stays;
+    uint32_t fill = stays < 32u ? m >> stays << stays : 0u;   // stayers that may fill a hole, the next one on top
+    uint32_t rank = 0;                                        // of the next hole's mover
+    auto place = [&](uint32_t q, uint32_t at) {
+        if (q < n)
+            rk[perm[a + q]] = at;
+        else
+            epos[e0 + q - n] = at;
+    };
+    for (uint32_t q = 0; q < len; ++q) {
+        const bool stay = m >> q & 1u;
+        if (stay && q < stays) {
+            place(q, q);
+        } else if (q < stays) {
+            const uint32_t from = 31u - (uint32_t) __builtin_clz(fill);
+            fill ^= 1u << from;
+            rk[perm[a + q]] = rank;
+            rank = len - from;
+            place(from, q);
+        } else if (!stay) {
+            rk[perm[a + q]] = q > stays ? len - q : rank;
+        }
+    }
+}
+
+// The listed cells, or all (list == nullptr).
+__global__ __launch_bounds__(64 * kBucketBlock) void k_ref_bucket(uint32_t ncells, const uint32_t *__restrict__ list,
+                                                                  const uint32_t *__restrict__ ostart,
                                                                   const uint32_t *__restrict__ perm,
                                                                   const uint32_t *__restrict__ gnew,
                                                                   const uint32_t *__restrict__ eoff,
                                                                   uint32_t *__restrict__ work,
                                                                   uint32_t *__restrict__ rk,
-                                                                  uint32_t *__restrict__ epos,
-                                                                  uint32_t *__restrict__ nstay)
+                                                                  uint32_t *__restrict__ epos, uint32_t *nstay)
 {
     constexpr uint32_t kThreads = 64 * kBucketBlock, kItems = 4;
     __shared__ uint32_t s_hole[kThreads], s_right[kThreads];
     __shared__ uint32_t s_part[kBucketBlock], s_holes;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    const uint32_t c0 = blockIdx.x * kBucketBlock;
-    if (const uint32_t c = c0 + wave; c < ncells) {
-        const uint32_t a = ostart[c], n = ostart[c + 1] - a;
-        const uint32_t e0 = eoff[c], len = n + (eoff[c + 1] - e0);
-        if (len <= 64u) {
-            const uint32_t e = lane < n ? perm[a + lane] : 0u;
-            const bool in = lane < len, stay = in && (lane >= n || gnew[e] == c);
-            const uint64_t m = __ballot(stay);
-            const uint32_t stays = (uint32_t) __popcll(m);
-            const uint32_t before = (uint32_t) __popcll(m & ((1ull << lane) - 1ull));
-            const uint32_t right = stays - before - 1u;   // a stayer's number from the right
-            const uint32_t holes = stays - (uint32_t) __popcll(stays < 64u ? m & ((1ull << stays) - 1ull) : m);
-            uint32_t *hole = s_hole + 64u * wave, *from = s_right + 64u * wave;
-            if (in && !stay && lane < stays) hole[lane - before] = lane;
-            if (stay && lane >= stays) from[right] = lane;
-            __builtin_amdgcn_wave_barrier();
-            if (stay) {
-                const uint32_t q = lane < stays ? lane : hole[right];
-                if (lane < n)
-                    rk[e] = q;
-                else
-                    epos[e0 + lane - n] = q;
-            } else if (in) {
-                const uint32_t h = lane < stays ? lane - before : holes;
-                rk[e] = lane > stays ? len - lane : h ? len - from[h - 1u] : 0u;
-            }
-            if (lane == 0u) nstay[c] = stays;
-        }
-    }
-    for (uint32_t u = 0; u < kBucketBlock && c0 + u < ncells; ++u) {
-        const uint32_t c = c0 + u;
-        const uint32_t a = ostart[c], n = ostart[c + 1] - a;
-        const uint32_t e0 = eoff[c], len = n + (eoff[c + 1] - e0);
-        if (len <= 64u) continue;
-        uint32_t *w = work + a + e0;   // hole h at h, the j-th stayer from the right at len - 1 - j
-        auto sum = [&](uint32_t v) {   // inclusive, over the workgroup's threads; the total in s_part
-            for (uint32_t d = 1; d < 64u; d <<= 1) {
-                const uint32_t o = (uint32_t) __shfl_up((int) v, d);
-                v += lane >= d ? o : 0u;
-            }
-            __syncthreads();
-            if (lane == 63u) s_part[wave] = v;
-            __syncthreads();
-            for (uint32_t g = 0; g < wave; ++g) v += s_part[g];
-            return v;
-        };
-        auto total = [&]() {
-            uint32_t t = 0;
-            for (uint32_t g = 0; g < kBucketBlock; ++g) t += s_part[g];
-            return t;
-        };
-        uint32_t mine = 0;
-        for (uint32_t q = tid; q < n; q += kThreads) mine += gnew[perm[a + q]] == c;
-        sum(mine);
-        const uint32_t stays = total() + (len - n);
-        if (tid == 0u) {
-            nstay[c] = stays;
-            s_holes = 0u;
-        }
-        uint32_t base = 0;   // stayers before the chunk
-        for (uint32_t q0 = 0; q0 < len; q0 += kThreads * kItems) {
-            const uint32_t q1 = q0 + kItems * tid;
-            uint32_t e[kItems];
-            bool stay[kItems];
-            uint32_t cnt = 0;
-#pragma unroll
-            for (uint32_t v = 0; v < kItems; ++v) e[v] = q1 + v < n ? perm[a + q1 + v] : 0u;
-#pragma unroll
-            for (uint32_t v = 0; v < kItems; ++v) {
-                stay[v] = q1 + v < len && (q1 + v >= n || gnew[e[v]] == c);
-                cnt += stay[v];
-            }
-            uint32_t before = base + sum(cnt) - cnt;
-            base += total();
-#pragma unroll
-            for (uint32_t v = 0; v < kItems; ++v) {
-                const uint32_t q = q1 + v;
-                if (q == stays) s_holes = stays - before;
-                if (stay[v]) {
-                    if (q >= stays)
-                        w[len - stays + before] = q;
-                    else if (q < n)
-                        rk[e[v]] = q;
+    const uint32_t m = list ? nstay[ncells] : ncells;
+    for (uint32_t c0 = blockIdx.x * kBucketBlock; c0 < m; c0 += gridDim.x * kBucketBlock) {
+        if (c0 + wave < m) {
+            const uint32_t c = list ? list[c0 + wave] : c0 + wave;
+            const uint32_t a = ostart[c], n = ostart[c + 1] - a;
+            const uint32_t e0 = eoff[c], len = n + (eoff[c + 1] - e0);
+            if (len <= 64u) {
+                const uint32_t e = lane < n ? perm[a + lane] : 0u;
+                const bool in = lane < len, stay = in && (lane >= n || gnew[e] == c);
+                const uint64_t ms = __ballot(stay);
+                const uint32_t stays = (uint32_t) __popcll(ms);
+                const uint32_t before = (uint32_t) __popcll(ms & ((1ull << lane) - 1ull));
+                const uint32_t right = stays - before - 1u;   // a stayer's number from the right
+                const uint32_t holes = stays - (uint32_t) __popcll(stays < 64u ? ms & ((1ull << stays) - 1ull) : ms);
+                uint32_t *hole = s_hole + 64u * wave, *from = s_right + 64u * wave;
+                if (in && !stay && lane < stays) hole[lane - before] = lane;
+                if (stay && lane >= stays) from[right] = lane;
+                __builtin_amdgcn_wave_barrier();
+                if (stay) {
+                    const uint32_t q = lane < stays ? lane : hole[right];
+                    if (lane < n)
+                        rk[e] = q;
                     else
-                        epos[e0 + q - n] = q;
-                } else if (q < len) {
-                    if (q < stays)
-                        w[q - before] = q;
-                    else if (q > stays)
-                        rk[e[v]] = len - q;
+                        epos[e0 + lane - n] = q;
+                } else if (in) {
+                    const uint32_t h = lane < stays ? lane - before : holes;
+                    rk[e] = lane > stays ? len - lane : h ? len - from[h - 1u] : 0u;
                 }
-                before += stay[v];
+                if (lane == 0u) nstay[c] = stays;
             }
         }
-        __syncthreads();
-        const uint32_t holes = s_holes;
-        for (uint32_t h = tid; h < holes; h += kThreads) {
-            const uint32_t hole = w[h], from = w[len - 1u - h];
-            rk[perm[a + hole]] = h ? len - w[len - h] : 0u;
-            if (from < n)
-                rk[perm[a + from]] = hole;
-            else
-                epos[e0 + from - n] = hole;
+        for (uint32_t u = 0; u < kBucketBlock && c0 + u < m; ++u) {
+            const uint32_t c = list ? list[c0 + u] : c0 + u;
+            const uint32_t a = ostart[c], n = ostart[c + 1] - a;
+            const uint32_t e0 = eoff[c], len = n + (eoff[c + 1] - e0);
+            if (len <= 64u) continue;
+            uint32_t *w = work + a + e0;   // hole h at h, the j-th stayer from the right at len - 1 - j
+            auto sum = [&](uint32_t v) {   // inclusive, over the workgroup's threads; the total in s_part
+                for (uint32_t d = 1; d < 64u; d <<= 1) {
+                    const uint32_t o = (uint32_t) __shfl_up((int) v, d);
+                    v += lane >= d ? o : 0u;
+                }
+                __syncthreads();
+                if (lane == 63u) s_part[wave] = v;
+                __syncthreads();
+                for (uint32_t g = 0; g < wave; ++g) v += s_part[g];
+                return v;
+            };
+            auto total = [&]() {
+                uint32_t t = 0;
+                for (uint32_t g = 0; g < kBucketBlock; ++g) t += s_part[g];
+                return t;
+            };
+            uint32_t mine = 0;
+            for (uint32_t q = tid; q < n; q += kThreads) mine += gnew[perm[a + q]] == c;
+            sum(mine);
+            const uint32_t stays = total() + (len - n);
+            if (tid == 0u) {
+                nstay[c] = stays;
+                s_holes = 0u;
+            }
+            uint32_t base = 0;   // stayers before the chunk
+            for (uint32_t q0 = 0; q0 < len; q0 += kThreads * kItems) {
+                const uint32_t q1 = q0 + kItems * tid;
+                uint32_t e[kItems];
+                bool stay[kItems];
+                uint32_t cnt = 0;
+#pragma unroll
+                for (uint32_t v = 0; v < kItems; ++v) e[v] = q1 + v < n ? perm[a + q1 + v] : 0u;
+#pragma unroll
+                for (uint32_t v = 0; v < kItems; ++v) {
+                    stay[v] = q1 + v < len && (q1 + v >= n || gnew[e[v]] == c);
+                    cnt += stay[v];
+                }
+                uint32_t before = base + sum(cnt) - cnt;
+                base += total();
+#pragma unroll
+                for (uint32_t v = 0; v < kItems; ++v) {
+                    const uint32_t q = q1 + v;
+                    if (q == stays) s_holes = stays - before;
+                    if (stay[v]) {
+                        if (q >= stays)
+                            w[len - stays + before] = q;
+                        else if (q < n)
+                            rk[e[v]] = q;
+                        else
+                            epos[e0 + q - n] = q;
+                    } else if (q < len) {
+                        if (q < stays)
+                            w[q - before] = q;
+                        else if (q > stays)
+                            rk[e[v]] = len - q;
+                    }
+                    before += stay[v];
+                }
+            }
+            __syncthreads();
+            const uint32_t holes = s_holes;
+            for (uint32_t h = tid; h < holes; h += kThreads) {
+                const uint32_t hole = w[h], from = w[len - 1u - h];
+                rk[perm[a + hole]] = h ? len - w[len - h] : 0u;
+                if (from < n)
+                    rk[perm[a + from]] = hole;
+                else
+                    epos[e0 + from - n] = hole;
+            }
+            if (tid == 0u && stays < n) {
+                const uint32_t e = perm[a + stays];
+                if (gnew[e] != c) rk[e] = holes ? len - w[len - holes] : 0u;
+            }
+            __syncthreads();
         }
-        if (tid == 0u && stays < n) {
-            const uint32_t e = perm[a + stays];
-            if (gnew[e] != c) rk[e] = holes ? len - w[len - holes] : 0u;
-        }
-        __syncthreads();
     }
 }
 
@@ -2515,11 +2577,23 @@ void launch_ref_counts(const RefBuffers &r, const uint32_t *gold, const uint32_t
     launch_exclusive_scan(r.n_depart, ncells + 1, r.partials, st);
 }
 
-void launch_ref_bucket(const RefBuffers &r, uint32_t ncells, const uint32_t *ostart, const uint32_t *perm,
+void launch_ref_bucket(const RefBuffers &r, uint32_t n, uint32_t ncells, const uint32_t *ostart, const uint32_t *perm,
                        const uint32_t *gnew, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_ref_bucket, dim3(blocks_for(ncells, kBucketBlock)), dim3(64 * kBucketBlock), 0, st, ncells, ostart, perm, gnew,
-                       (const uint32_t *) r.n_early, r.work, r.rk, r.epos, r.nstay);
+    const uint32_t *eoff = r.n_early;
+    if (ncells <= kBucketWaveCells) {
+        hipLaunchKernelGGL(k_ref_bucket, dim3(blocks_for(ncells, kBucketBlock)), dim3(64 * kBucketBlock), 0, st, ncells,
+                           (const uint32_t *) nullptr, ostart, perm, gnew, eoff, r.work, r.rk, r.epos, r.nstay);
+        return;
+    }
+    uint32_t *list = r.mkey;   // free until the movers are written; the buckets hold at most 2 n entries in all
+    hipLaunchKernelGGL(k_ref_bucket_lanes, dim3(blocks_for(ncells, 256)), dim3(256), 0, st, ncells, ostart, perm, gnew,
+                       eoff, list, r.rk, r.epos, r.nstay);
+    const uint32_t most = (uint32_t) (2ull * n / (kLaneBucket + 1));
+    if (most)
+        hipLaunchKernelGGL(k_ref_bucket, dim3(std::min(blocks_for(most, kBucketBlock), 2048u)),
+                           dim3(64 * kBucketBlock), 0, st, ncells, (const uint32_t *) list, ostart, perm, gnew, eoff,
+                           r.work, r.rk, r.epos, r.nstay);
 }
 
 void launch_ref_movers(const RefBuffers &r, const uint32_t *gold, const uint32_t *gnew, uint32_t n, uint32_t ncells,
