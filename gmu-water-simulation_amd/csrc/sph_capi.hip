@@ -1319,9 +1319,13 @@ struct Snapshot {
         SPH_HIP(hipMemcpyAsync(c->table_d, table.data(), table.size() * sizeof(sph::Scene), hipMemcpyHostToDevice,
                                c->stream));
         SPH_TRY(clear_counts(c));
+        // the saved keys' counts are taken again: the next step starts as the saved one would have
+        if (keys_valid && c->by_counts) {
+            sph::launch_hash(c->soa(cur, id_cur), c->key_h, c->counts(), c->table(), c->k.h, c->stream);
+            SPH_TRY(launch_error("hash launch"));
+        }
         SPH_HIP(hipStreamSynchronize(c->stream));
-        // the counts of the saved keys are gone: the next step hashes again
-        c->keys_valid = keys_valid && !c->by_counts;
+        c->keys_valid = keys_valid;
         c->steps_done = steps_done;
         c->counts_stale = !c->emit_h.empty();
         return SPH_OK;
