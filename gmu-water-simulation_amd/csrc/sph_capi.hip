@@ -1831,11 +1831,14 @@ sph_status sph_autotune(sph_ctx *c, uint32_t steps, float *ms_out)
         c->fault_at_step = -1;
         Snapshot snap{c};
         sph_status st = snap.save();
-        int best_v = c->variant, best_m = c->nb_mode;
+        const int own_v = c->variant;
+        int best_v = own_v, best_m = c->nb_mode;
         float best = -1.0f;
         for (int mode = 0; mode < kModes && !st; ++mode) {
             if (mode == SPH_NEIGHBOURS_LISTS && c->kmax == 0) continue;
-            for (int v = 0; v < sph::kNumVariants && !st; ++v) {
+            // the shared-particle kernels have one shape: timed once, and no reason to change the variant
+            const bool one_shape = mode == SPH_NEIGHBOURS_MASKS && c->split;
+            for (int v = one_shape ? own_v : 0; v < (one_shape ? own_v + 1 : sph::kNumVariants) && !st; ++v) {
                 st = snap.restore();
                 if (st) break;
                 c->variant = v;
@@ -1852,7 +1855,9 @@ sph_status sph_autotune(sph_ctx *c, uint32_t steps, float *ms_out)
                     st = fail(SPH_ERR_HIP, "hipEventElapsedTime");
                 if (st) break;
                 ms /= (float) steps;
-                if (ms_out) ms_out[kModes * v + mode] = ms;
+                if (ms_out)
+                    for (int w = one_shape ? 0 : v; w < (one_shape ? sph::kNumVariants : v + 1); ++w)
+                        ms_out[kModes * w + mode] = ms;
                 if (best < 0.0f || ms < best) {
                     best = ms;
                     best_v = v;

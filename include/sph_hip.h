@@ -336,7 +336,9 @@ sph_status sph_variant_shape(int variant, int *threads, int *unroll, int *pairs,
 /* Times `steps` steps of every (variant, neighbour mode) choice from the current state,
  * keeps the fastest and restores the state, so the call changes nothing but the choice.
  * ms_out (may be NULL) receives 3*SPH_NUM_VARIANTS ms-per-step figures, index
- * 3*variant + mode, negative where a choice was not run. */
+ * 3*variant + mode, negative where a choice was not run. Up to 40,960 slots in use
+ * SPH_NEIGHBOURS_MASKS has one shape: it is timed once for all variants, and where it is
+ * the fastest the variant stays as it is. */
 sph_status sph_autotune(sph_ctx *ctx, uint32_t steps, float *ms_out);
 
 /* ------------------------------------------------------------------------------

@@ -32,3 +32,23 @@ def test_the_next_step_starts_as_before(hip):
     assert_bits_equal(a.download()[0], b.download()[0], "positions after the autotuner")
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("variant", [3, 12])
+def test_one_shape_keeps_the_variant(hip, variant):
+    """Up to 40,960 slots the mask mode has one kernel for all variants: one time stands
+    for all, and where it wins the variant stays what it was."""
+    lib = hip._lib
+    pos = hip.scenes.lattice(12, 12, 12, 0.4, jitter_h=0.01, seed=4)
+    with hip.SceneBatch([(0.4, len(pos))]) as b:
+        b.upload(0, pos)
+        b.set_variant(variant, lib.NEIGHBOURS_MASKS)
+        b.step(2)
+        times = b.autotune(steps=2)
+        masks = [times[(v, lib.NEIGHBOURS_MASKS)] for v in range(lib.NUM_VARIANTS)]
+        assert len(set(masks)) == 1
+        chosen, mode = b.variant()
+        if mode == lib.NEIGHBOURS_MASKS:
+            assert chosen == variant
+        else:
+            assert times[(chosen, mode)] < masks[0]
