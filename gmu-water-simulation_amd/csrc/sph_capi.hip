@@ -155,10 +155,9 @@ struct sph_ctx {
     uint32_t up_cap = 0;
 
     // readback: pinned host buffers the device writes by id, its flag behind the
-    // positions, and (device) each id's slot
+    // positions (each id's slot: key_t, which only the grid phase uses)
     float *rb_pos = nullptr, *rb_vel = nullptr;
     size_t rb_cap = 0;
-    uint32_t *rb_at = nullptr;
 
     // profiling
     hipEvent_t ev[kProfileSlots][2] = {};
@@ -1370,9 +1369,9 @@ uint64_t sph_slot_bytes(uint32_t max_neighbours)
     const uint64_t lists = max_neighbours == SPH_NEIGHBOUR_LISTS_OFF ? 0 : max_neighbours;
     // pos/vel ping-pong 48, ids 8, keys and values 20, rho 4, records 32,
     // accelerations 12, counts 8, row masks (the default mode without
-    // lists), list entries, 4 for the readback's slots by id, and 8 for the
-    // histograms, the group map and the scene's share of the cell table and counts
-    return 48 + 8 + 20 + 4 + 4 * sph::kRecWords + 12 + 8 + (lists ? 4 * lists : 9 * 4 * sph::kMaskWords) + 4 + 8;
+    // lists), list entries, and 12 for the histograms, the group map and the scene's
+    // share of the cell table and counts
+    return 48 + 8 + 20 + 4 + 4 * sph::kRecWords + 12 + 8 + (lists ? 4 * lists : 9 * 4 * sph::kMaskWords) + 12;
 }
 
 int sph_grid_res(float box)
@@ -1891,18 +1890,15 @@ sph_status sph_scene_readback(sph_ctx *c, uint32_t scene, int with_velocity, con
             const size_t cap = std::max<size_t>(std::max<size_t>(n, c->rb_cap), 1);
             if (c->rb_pos) (void) hipHostFree(c->rb_pos);
             if (c->rb_vel) (void) hipHostFree(c->rb_vel);
-            dfree(c, c->rb_at);
             c->rb_pos = c->rb_vel = nullptr;
-            c->rb_at = nullptr;
             c->rb_cap = 0;
             SPH_HIP(hipHostMalloc((void **) &c->rb_pos, cap * 12 + 4, hipHostMallocDefault));
             if (with_velocity) SPH_HIP(hipHostMalloc((void **) &c->rb_vel, cap * 12, hipHostMallocDefault));
-            SPH_TRY(dalloc(c, &c->rb_at, cap));
             c->rb_cap = cap;
         }
         volatile uint32_t *bad = (volatile uint32_t *) (c->rb_pos + 3 * c->rb_cap);
         *bad = 0;
-        sph::launch_pack_by_id(c->soa(c->cur, c->id_cur), s.poff, n, c->rb_at, c->rb_pos,
+        sph::launch_pack_by_id(c->soa(c->cur, c->id_cur), s.poff, n, c->key_t, c->rb_pos,
                                with_velocity ? c->rb_vel : nullptr, (uint32_t *) bad, c->stream);
         SPH_TRY(launch_error("readback launch"));
         SPH_HIP(hipStreamSynchronize(c->stream));

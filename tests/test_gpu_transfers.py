@@ -1,8 +1,12 @@
 """Particles in and out at the edges of the transfers' parts: 256 particles a
 workgroup, four words a piece, 16,384 particles an upload's part; at rest or moving,
 with the ids that upload gives or shuffled ones, appended behind others."""
+import ctypes as C
+
 import numpy as np
 import pytest
+
+from test_zz_no_alloc import _hip_runtime
 
 pytestmark = pytest.mark.gpu
 
@@ -35,3 +39,34 @@ def test_upload_append_readback(hip, n, moving, shuffled):
         if ids[:n].max() >= n:
             with pytest.raises(Exception, match="ids are not 0..count-1"):
                 sim.readback()
+
+
+def test_readback_takes_no_device_memory(hip):
+    """The slots by id lie in a buffer that the context has: the first readback of 4 million
+    particles (16 MB of them) leaves the device's free memory as it was."""
+    free, total = C.c_size_t(), C.c_size_t()
+    rt = _hip_runtime()
+
+    def free_bytes():
+        assert rt.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        return free.value
+
+    n = 4_000_000
+    rng = np.random.default_rng(11)
+    pos = (9.0 * (rng.random((n, 3)) - 0.5)).astype(np.float32)
+    ids = rng.permutation(n).astype(np.uint32)
+    with hip.HIPGridParticleSimulator(10.0, capacity=n) as sim:
+        sim.upload(pos, None, ids)
+        sim.sync()
+        before = free_bytes()
+        p, _ = sim.readback()
+        after = free_bytes()
+        assert np.array_equal(p[ids].view(np.uint32), pos.view(np.uint32))
+        assert before - after < 4 * n
+        # between phases: the grid phase's results stay as they are
+        sim.updateGrid()
+        p, _ = sim.readback(with_velocity=False)
+        assert np.array_equal(p[ids].view(np.uint32), pos.view(np.uint32))
+        for phase in (sim.updateDensityPressure, sim.updateForces, sim.updateCollisions, sim.integrate):
+            phase()
+            assert np.isfinite(sim.readback()[0]).all()
