@@ -98,3 +98,44 @@ def test_sort_with_uneven_scenes_and_an_emitter(hip):
                 b.phase(phase)
             b.step(2)
         b.close()
+
+
+@pytest.mark.parametrize("n,run", [(256, 1), (258, 1), (2000, 1), (2000, 3), (2000, 7), (40000, 64), (5001, 1000)])
+def test_crowded_cells(hip, n, run):
+    """Two cells of n / 2 particles, as many as a lane goes through by itself (128), one more,
+    and many, with runs of 1 to 1,000 consecutive slots."""
+    lib = hip._lib
+    h = float(hip.scenes.H)
+    rng = np.random.default_rng([n, run])
+    pos = (0.01 * h * rng.random((n, 3)) + 0.3 * h).astype(np.float32)
+    pos[(np.arange(n) // run) % 2 == 1, 0] += np.float32(h)
+    print("%d particles, runs of %d" % (n, run), flush=True)
+    sim = hip.HIPGridParticleSimulator((4 * h, 3 * h, 3 * h), capacity=n + 3)
+    sim.upload(pos, rng.normal(0, 0.2, (n, 3)).astype(np.float32))
+    for step in range(2):
+        sim.updateGrid()
+        check_sorted(sim, lib, sim.grid_dims()[1])
+        for phase in (sim.updateDensityPressure, sim.updateForces, sim.updateCollisions, sim.integrate):
+            phase()
+    sim.close()
+
+
+def test_a_crowded_cell_does_not_hold_up_the_sort(hip):
+    """40,000 particles in one cell against as many in 8,000 cells: the sort's time grew with
+    the square of a cell's particles (14 times as long), and may be some times as long."""
+    h = float(hip.scenes.H)
+    n, box = 40000, 19.5 * h
+    rng = np.random.default_rng(1)
+    at = rng.random((n, 3))
+    ms = []
+    for pos in ((box * (at - 0.5)), 0.9 * h * at):
+        with hip.HIPGridParticleSimulator(box, capacity=n) as sim:
+            t = []
+            for _ in range(6):
+                sim.upload(pos.astype(np.float32))
+                t.append(sim.updateGrid())
+                for phase in (sim.updateDensityPressure, sim.updateForces, sim.updateCollisions, sim.integrate):
+                    phase()
+            ms.append(min(t[1:]))
+    print("spread %.3f ms, crowded %.3f ms" % tuple(ms), flush=True)
+    assert ms[1] < 6.0 * ms[0]
