@@ -113,6 +113,7 @@ struct sph_ctx {
     uint32_t ccount_cap = 0;
     bool by_counts = false;   // the layout's grid phase sorts by counts (else by digits)
     bool split = false;       // its neighbour passes share a particle between lanes (mask mode)
+    uint32_t *crowd = nullptr;   // unless its particles are crowded (NeighbourList)
     uint32_t *hist = nullptr;
     uint32_t *partials = nullptr;
     uint32_t *cstart = nullptr;
@@ -189,6 +190,7 @@ struct sph_ctx {
         nl.kmax = kmax;
         nl.mode = nb_mode == SPH_NEIGHBOURS_MASKS && split ? (int) sph::kNbSplit : nb_mode;
         nl.masks = masks;
+        nl.crowd = crowd;
         return nl;
     }
 
@@ -209,6 +211,9 @@ struct sph_ctx {
         cc.arr = val_t;
         return cc;
     }
+
+    // where the grid phase adds up the launch's crowding
+    uint32_t *crowding() const { return split ? crowd : nullptr; }
 
     bool ref_order() const { return (flags & SPH_FLAG_REFERENCE_ORDER) != 0; }
 
@@ -761,7 +766,8 @@ sph_status run_grid_reference(sph_ctx *c)
         StageTimer t(c, SPH_STAGE_CELLS);
         if (t.st) return t.st;
         sph::launch_ref_place(c->ref, c->key_s, c->val_s, n, C, c->cstart, c->stream);
-        sph::launch_ref_final(c->ref, c->key_h, c->cstart, c->key_s, c->val_s, c->ocell, tab, c->stream);
+        sph::launch_ref_final(c->ref, c->key_h, c->cstart, c->key_s, c->val_s, c->ocell, c->crowding(), tab,
+                              c->stream);
     }
     return SPH_OK;
 }
@@ -794,7 +800,7 @@ sph_status run_grid(sph_ctx *c)
         }
         StageTimer t(c, SPH_STAGE_REORDER);
         if (t.st) return t.st;
-        sph::launch_gather(cur, dst, c->key_t, c->key_s, c->cstart, c->val_s, tab, c->stream);
+        sph::launch_gather(cur, dst, c->key_t, c->key_s, c->cstart, c->val_s, c->crowding(), tab, c->stream);
     } else {
         if (c->ref_order()) {
             SPH_TRY(run_grid_reference(c));
@@ -807,6 +813,7 @@ sph_status run_grid(sph_ctx *c)
             StageTimer t(c, SPH_STAGE_CELLS);
             if (t.st) return t.st;
             sph::launch_cell_start(c->key_s, n, c->total_cells, c->cstart, c->stream);
+            if (c->split) sph::launch_crowding(c->key_s, c->cstart, c->crowd, tab, c->stream);
         }
         StageTimer t(c, SPH_STAGE_REORDER);
         if (t.st) return t.st;
@@ -1189,6 +1196,7 @@ sph_status alloc_buffers(sph_ctx *c, uint32_t max_segments)
     SPH_TRY(dalloc(c, &c->table_d, max_segments));
     SPH_TRY(dalloc(c, &c->group_d, (P + sph::kGroupSlots - 1) / sph::kGroupSlots));
     SPH_TRY(dalloc(c, &c->emit_d, c->scenes.size()));
+    SPH_TRY(dalloc(c, &c->crowd, sph::kCrowdWords));
     if (c->flags & SPH_FLAG_PROFILE)
         for (auto &pair : c->ev)
             for (auto &ev : pair)

@@ -59,6 +59,8 @@ constexpr uint32_t kMaskBits = kMaskWordBits * kMaskWords;
 constexpr uint32_t kSplitCap = 2u * 9u * kMaskWords;
 constexpr uint32_t kNbOverflow = 0xFFFFFFFFu;
 
+constexpr uint32_t kSplitSlots = 40960;
+
 // Whether the neighbour passes of a launch over `slots` slots, the widest scene of
 // `widest`, share each particle between four lanes (k_density_split, k_forces_split):
 // faster while one wave's time decides, slower once there are waves enough to fill the
@@ -68,8 +70,22 @@ constexpr uint32_t kNbOverflow = 0xFFFFFFFFu;
 // 83; four scenes of 16,000 96 and 82. (Entries are 16-bit slots.)
 inline bool split_neighbours(uint32_t slots, uint32_t widest)
 {
-    return widest <= 65536u && slots <= 40960u;
+    return widest <= 65536u && slots <= kSplitSlots;
 }
+
+// A launch that split_neighbours picks still takes the one-lane kernels' way (masks and
+// all, within the same launch) where its particles lie so close that pairs decide, not a
+// wave's latency: if a cell has more than kCrowdCell of them, or the particles' cells
+// together have more than kCrowdWork slots, each counted for every one of its particles
+// (about a quarter of the launch's pairs). The grid phase adds that up, a word for every
+// 256 slots (`crowd`); reading the words takes the two passes 0.3 to 0.8 us. Steps of
+// blocks at rest, us, shared and not: 40,000 particles at spacing h / 2.5 174 and 167,
+// h / 3 234 and 203, h / 4 504 and 421, h / 5 1,896 and 817; 15,000 at h / 3 192 and 192,
+// h / 4 403 and 396, h / 5 1,492 and 773; 3,375 at h / 3.5 258 and 277, h / 4 365 and 374,
+// h / 4.5 966 and 553 (more neighbours than the lists hold).
+constexpr uint32_t kCrowdCell = 64;
+constexpr uint32_t kCrowdWork = 800000;
+constexpr uint32_t kCrowdWords = kSplitSlots / 256;
 
 struct NeighbourList {
     uint32_t *idx;
@@ -77,6 +93,7 @@ struct NeighbourList {
     uint32_t kmax;
     int mode;            // NeighbourMode
     uint32_t *masks;     // mask mode: 32-bit words of accepted-candidate bits
+    uint32_t *crowd;     // kNbSplit: the launch's crowding
 };
 
 __host__ __device__ inline size_t list_slot(const NeighbourList &nl, uint32_t i)
@@ -204,7 +221,7 @@ void launch_ref_movers(const RefBuffers &r, const uint32_t *gold, const uint32_t
 void launch_ref_place(const RefBuffers &r, const uint32_t *skey, const uint32_t *sval, uint32_t n, uint32_t ncells,
                       uint32_t *start, hipStream_t st);
 void launch_ref_final(const RefBuffers &r, const uint32_t *gnew, const uint32_t *start, uint32_t *skey, uint32_t *perm,
-                      uint32_t *ocell, const SceneTable &t, hipStream_t st);
+                      uint32_t *ocell, uint32_t *crowd, const SceneTable &t, hipStream_t st);
 
 // The grid phase from the keys and their counts (canonical order), in three steps.
 // 1. The cell table, the counts' exclusive scan: start[c] = the first sorted slot
@@ -213,18 +230,22 @@ void launch_ref_final(const RefBuffers &r, const uint32_t *gnew, const uint32_t 
 // 2. Every slot to its cell's range, in no particular order (list), and the sorted
 //    keys; the counts and the state are zeroed for the next step.
 // 3. The particles to their places, a stable sort by key, and the permutation.
-// Nothing is written for unused slots in 2 and 3.
+// Nothing is written for unused slots in 2 and 3. crowd: the launch's crowding
+// (NeighbourList), written in 3, or null.
 __host__ __device__ inline uint32_t scan_state_words(uint32_t ncells) { return scan_blocks(ncells + 1) + 1; }
 void launch_cell_table(const CellCount &cc, unsigned long long *state, uint32_t *start, uint32_t ncells, hipStream_t st,
                        uint32_t poll_limit = kScanPollLimit);
 void launch_place(const uint32_t *key, const CellCount &cc, unsigned long long *state, const uint32_t *start,
                   uint32_t ncells, uint32_t *list, uint32_t *skey, const SceneTable &t, hipStream_t st);
 void launch_gather(const ParticleSoA &src, const ParticleSoA &dst, const uint32_t *list, const uint32_t *skey,
-                   const uint32_t *start, uint32_t *perm, const SceneTable &t, hipStream_t st);
+                   const uint32_t *start, uint32_t *perm, uint32_t *crowd, const SceneTable &t, hipStream_t st);
 
 // start[c] = first slot whose sorted key is >= c, c in [0, ncells].
 void launch_cell_start(const uint32_t *sorted_keys, uint32_t n, uint32_t ncells, uint32_t *start,
                        hipStream_t st);
+
+// The launch's crowding from the sorted keys.
+void launch_crowding(const uint32_t *skey, const uint32_t *start, uint32_t *crowd, const SceneTable &t, hipStream_t st);
 
 // dst[k] = src[perm[k]] for positions, velocities and ids.
 void launch_reorder(const ParticleSoA &src, const ParticleSoA &dst, const uint32_t *perm, uint32_t n,

@@ -756,6 +756,41 @@ __global__ __launch_bounds__(kTriples) void k_pack_by_id(ParticleSoA p, const ui
 // passes, the table from the sorted keys and the gather; 50,653 particles 15.0 us
 // against 39.2. The counting costs the force pass about 10 us at 1,048,576.
 
+// The sum of v over the wave's 64 lanes, all of them active.
+__device__ __forceinline__ uint32_t wave_sum(uint32_t v)
+{
+    int x = (int) v;
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);   // row_shr:1
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);   // row_bcast:15
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);   // row_bcast:31
+    return (uint32_t) __builtin_amdgcn_readlane(x, 63);
+}
+
+// The crowding (NeighbourList) of a workgroup's 256 slots from first, whose cells have m
+// slots (0 for slots without a particle). All threads take part.
+__device__ __forceinline__ void store_crowding(uint32_t *__restrict__ crowd, uint32_t first, uint32_t m)
+{
+    __shared__ uint32_t s_sum[4];
+    const uint32_t sum = __any(m > kCrowdCell) ? kCrowdWork + 1u : wave_sum(m);
+    s_sum[threadIdx.x >> 6] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0u) crowd[first / 256u] = s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
+}
+
+// The crowding where the grid phase does not come by it, from the sorted keys.
+__global__ __launch_bounds__(256) void k_crowding(const uint32_t *__restrict__ skey, const uint32_t *__restrict__ start,
+                                                  uint32_t *__restrict__ crowd, SceneTable t)
+{
+    const uint32_t first = blockIdx.x * 256u, i = first + threadIdx.x;
+    const Scene s = block_scene(t, first);
+    uint32_t m = 0;
+    if (i < t.nslots && i - s.poff < s.n) m = start[skey[i] + 1u] - start[skey[i]];
+    store_crowding(crowd, first, m);
+}
+
 // list[start[key] + arr] = slot, and the sorted keys (one cell's are all the same).
 // Clears the counts and the scan's words, which the scan has read.
 __global__ __launch_bounds__(256) void k_place(const uint32_t *__restrict__ key, CellCount cc,
@@ -822,15 +857,15 @@ __device__ __forceinline__ uint32_t slots_below(const uint32_t *__restrict__ lis
 }
 
 // The particle at list[q] moves to its place in the cell: after the cell's slots
-// that come before it in the old order. In a cell of up to kCrowd slots every lane goes
+// that come before it in the old order. In a cell of up to kManySlots every lane goes
 // through the cell by itself, in a larger one the wave does (slots_below): the grid phase
 // of 100,000 particles in eight cells takes 0.70 ms (lanes by themselves 2.72), in one
 // cell 0.45 (3.49), of 2,000 in one cell 79 us (130), and as before in ordinary cells.
-constexpr uint32_t kCrowd = 128;
+constexpr uint32_t kManySlots = 128;
 
 __global__ __launch_bounds__(256) void k_gather(ParticleSoA src, ParticleSoA dst, const uint32_t *__restrict__ list,
                                                 const uint32_t *__restrict__ skey, const uint32_t *__restrict__ start,
-                                                uint32_t *__restrict__ perm, SceneTable t)
+                                                uint32_t *__restrict__ perm, uint32_t *__restrict__ crowd, SceneTable t)
 {
     __shared__ uint32_t s_slot[256], s_count[256];
     const uint32_t first = xcd_block(blockIdx.x, gridDim.x) * 256u, q = first + threadIdx.x;
@@ -851,20 +886,21 @@ __global__ __launch_bounds__(256) void k_gather(ParticleSoA src, ParticleSoA dst
         vz = src.vz[i];
         id = src.id[i];
     }
+    if (crowd) store_crowding(crowd, first, b - a);
     uint32_t d = a;
-    const bool crowd = b - a > kCrowd;
-    if (!crowd) {
+    const bool many = b - a > kManySlots;
+    if (!many) {
         uint32_t e = a;
         for (; e + 4u <= b; e += 4u)
             d += (uint32_t) (list[e] < i) + (uint32_t) (list[e + 1] < i) + (uint32_t) (list[e + 2] < i) +
                  (uint32_t) (list[e + 3] < i);
         for (; e < b; ++e) d += (uint32_t) (list[e] < i);
     }
-    for (uint64_t left = __ballot(crowd); left;) {   // crowded cell by crowded cell of the wave
+    for (uint64_t left = __ballot(many); left;) {   // cell by cell of the wave
         const int lead = (int) __builtin_ctzll(left);
         const uint32_t a0 = (uint32_t) __builtin_amdgcn_readlane((int) a, lead);
         const uint32_t b0 = (uint32_t) __builtin_amdgcn_readlane((int) b, lead), wave = threadIdx.x & 192u;
-        const bool mine = crowd && a == a0;
+        const bool mine = many && a == a0;
         const uint32_t below = slots_below(list, a0, b0, i, mine, s_slot + wave, s_count + wave);
         if (mine) d += below;
         left &= ~__ballot(mine);
@@ -1212,12 +1248,14 @@ __global__ __launch_bounds__(256) void k_ref_counts(const uint32_t *__restrict__
 __global__ __launch_bounds__(256) void k_ref_final(const uint32_t *__restrict__ gnew, const uint32_t *__restrict__ rk,
                                                    const uint32_t *__restrict__ start, uint32_t *__restrict__ skey,
                                                    uint32_t *__restrict__ perm, uint32_t *__restrict__ ocell,
-                                                   SceneTable t)
+                                                   uint32_t *__restrict__ crowd, SceneTable t)
 {
     const uint32_t first = blockIdx.x * 256u, i = first + threadIdx.x;
     const Scene s = block_scene(t, first);
+    const uint32_t c = i < t.nslots ? gnew[i] : 0u, at = start[c];
+    if (crowd) store_crowding(crowd, first, i < t.nslots && i - s.poff < s.n ? start[c + 1u] - at : 0u);
     if (i >= t.nslots) return;
-    const uint32_t c = gnew[i], f = start[c] + rk[i];   // < nslots by construction
+    const uint32_t f = at + rk[i];   // < nslots by construction
     if (f >= t.nslots) return;
     skey[f] = c;
     perm[f] = i;
@@ -1276,6 +1314,20 @@ __device__ __forceinline__ float4 ld4(__amdgpu_buffer_rsrc_t r, uint32_t byte_of
 {
     return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, (int) byte_off, 0, 0));
 }
+
+// Whether a launch over n slots is crowded (NeighbourList): each lane's words, and their
+// sum, apart so that other loads can be issued between the two.
+__device__ __forceinline__ uint32_t crowd_word(const uint32_t *crowd, uint32_t n)
+{
+    static_assert(kCrowdWords <= 192, "three words a lane");
+    const __amdgpu_buffer_rsrc_t r = rsrc(crowd, (n + 255u) / 256u * 4u);   // 0 past the last word
+    const int at = (int) (threadIdx.x & 63u) * 4;
+    return (uint32_t) __builtin_amdgcn_raw_buffer_load_b32(r, at, 0, 0) +
+           (uint32_t) __builtin_amdgcn_raw_buffer_load_b32(r, at + 256, 0, 0) +
+           (uint32_t) __builtin_amdgcn_raw_buffer_load_b32(r, at + 512, 0, 0);
+}
+
+__device__ __forceinline__ bool is_crowded(uint32_t word) { return wave_sum(word) > kCrowdWork; }
 
 __device__ __forceinline__ uint2 ld2u(__amdgpu_buffer_rsrc_t r, uint32_t byte_off)
 {
@@ -1498,20 +1550,13 @@ __device__ __forceinline__ void store_density(const DensityFields &f, const Part
 // (masks, and nl.cnt[i] = 1 when a run is too long for them); with kDiag, the
 // accepted count. T threads per workgroup, U candidates per lane per trip.
 template <int T, int U, bool kLists, bool kMasks, bool kDiag, bool kRef>
-__global__ __launch_bounds__(T) void k_density(ParticleSoA p, const uint32_t *__restrict__ cell,
-                                               const uint32_t *__restrict__ start, DensityFields f,
-                                               NeighbourList nl, uint32_t *__restrict__ masks, SceneTable t,
-                                               Consts k)
+__device__ __forceinline__ void density_of(const ParticleSoA &p, const uint32_t *__restrict__ cell,
+                                           const uint32_t *__restrict__ start, const DensityFields &f,
+                                           const NeighbourList &nl, uint32_t *__restrict__ masks, const Scene &s,
+                                           const Consts &k, uint32_t i, float *my)
 {
-    static_assert(kMaskWordBits % U == 0, "a trip must not straddle two mask words");
-    static_assert(kGroupSlots % T == 0, "a workgroup must lie in one slot group");
     constexpr int kCap = density_list_cap<U>();
-    __shared__ float lst[kCap * T];
-    const uint32_t first = xcd_block(blockIdx.x, gridDim.x) * (uint32_t) T, i = first + threadIdx.x;
-    const Scene s = block_scene(t, first);
     const uint32_t li = i - s.poff;
-    if (i >= t.nslots || li >= s.n) return;
-    float *my = lst + threadIdx.x;
     uint32_t *nidx = kLists ? nl.idx + list_slot(nl, i) : nullptr;
     const BufView bv = buf_view(p, f, s);
     const float xi = p.px[i], yi = p.py[i], zi = p.pz[i];
@@ -1558,6 +1603,21 @@ __global__ __launch_bounds__(T) void k_density(ParticleSoA p, const uint32_t *__
     if (kLists) nl.cnt[i] = nn;
     if (kMasks) nl.cnt[i] = rec_masks.overflow ? 1u : 0u;
     if (kDiag) f.ncount[i] = nc;
+}
+
+template <int T, int U, bool kLists, bool kMasks, bool kDiag, bool kRef>
+__global__ __launch_bounds__(T) void k_density(ParticleSoA p, const uint32_t *__restrict__ cell,
+                                               const uint32_t *__restrict__ start, DensityFields f,
+                                               NeighbourList nl, uint32_t *__restrict__ masks, SceneTable t,
+                                               Consts k)
+{
+    static_assert(kMaskWordBits % U == 0, "a trip must not straddle two mask words");
+    static_assert(kGroupSlots % T == 0, "a workgroup must lie in one slot group");
+    __shared__ float lst[density_list_cap<U>() * T];
+    const uint32_t first = xcd_block(blockIdx.x, gridDim.x) * (uint32_t) T, i = first + threadIdx.x;
+    const Scene s = block_scene(t, first);
+    if (i >= t.nslots || i - s.poff >= s.n) return;
+    density_of<T, U, kLists, kMasks, kDiag, kRef>(p, cell, start, f, nl, masks, s, k, i, lst + threadIdx.x);
 }
 
 struct ForceSums {
@@ -2108,6 +2168,24 @@ constexpr int phase_threads()
 }
 
 template <bool kRef, bool kMasks>
+__device__ __forceinline__ void phase_of(const ParticleSoA &p, const uint32_t *__restrict__ cell,
+                                         const uint32_t *__restrict__ start, const DensityFields &f,
+                                         const NeighbourList &nl, float *__restrict__ ax, float *__restrict__ ay,
+                                         float *__restrict__ az, const SceneTable &t, const Scene &s, const Consts &k,
+                                         uint32_t i, uint32_t *my)
+{
+    const uint32_t li = i - s.poff;
+    if (i >= t.nslots || li >= s.n) return;
+    float a0, a1, a2;
+    sph_accel<kRef, phase_threads<kMasks>(), kPhaseUnroll, kMasks>(p, cell, start, f, nl, my, i, li, s, k, p.px[i],
+                                                                   p.py[i], p.pz[i], p.vx[i], p.vy[i], p.vz[i], a0,
+                                                                   a1, a2);
+    ax[i] = a0;
+    ay[i] = a1;
+    az[i] = a2;
+}
+
+template <bool kRef, bool kMasks>
 __global__ __launch_bounds__(phase_threads<kMasks>()) void k_forces(ParticleSoA p, const uint32_t *__restrict__ cell,
                                                                     const uint32_t *__restrict__ start,
                                                                     DensityFields f, NeighbourList nl,
@@ -2116,16 +2194,9 @@ __global__ __launch_bounds__(phase_threads<kMasks>()) void k_forces(ParticleSoA 
 {
     constexpr int T = phase_threads<kMasks>();
     __shared__ uint32_t lst[(kMasks ? 2 * kPhaseWords + 2 : kListCap) * T];
-    const uint32_t first = xcd_block(blockIdx.x, gridDim.x) * (uint32_t) T, i = first + threadIdx.x;
+    const uint32_t first = xcd_block(blockIdx.x, gridDim.x) * (uint32_t) T;
     const Scene s = block_scene(t, first);
-    const uint32_t li = i - s.poff;
-    if (i >= t.nslots || li >= s.n) return;
-    float a0, a1, a2;
-    sph_accel<kRef, T, kPhaseUnroll, kMasks>(p, cell, start, f, nl, lst + threadIdx.x, i, li, s, k, p.px[i], p.py[i],
-                                             p.pz[i], p.vx[i], p.vy[i], p.vz[i], a0, a1, a2);
-    ax[i] = a0;
-    ay[i] = a1;
-    az[i] = a2;
+    phase_of<kRef, kMasks>(p, cell, start, f, nl, ax, ay, az, t, s, k, first + threadIdx.x, lst + threadIdx.x);
 }
 
 __global__ __launch_bounds__(256) void k_collide(ParticleSoA p, float *__restrict__ ax, float *__restrict__ ay,
@@ -2170,22 +2241,15 @@ __global__ __launch_bounds__(256) void k_integrate(ParticleSoA p, const float *_
 // a wave at a time (wave_list_sums); kNbMasks iterates the density pass's row
 // masks (mask_sums). Particles whose list or masks overflowed walk their cells.
 template <int T, int U, int C, int kStall, bool kQueue, int kMode, bool kStoreAcc, bool kRef>
-__global__ __launch_bounds__(T) void k_forces_fused(ParticleSoA p, const uint32_t *__restrict__ cell,
-                                                    const uint32_t *__restrict__ start, DensityFields f,
-                                                    NeighbourList nl, ParticleSoA out,
-                                                    uint32_t *__restrict__ key_next, CellCount cc,
-                                                    float *__restrict__ ax, float *__restrict__ ay,
-                                                    float *__restrict__ az, SceneTable t, Consts k)
+__device__ __forceinline__ void fused_of(const ParticleSoA &p, const uint32_t *__restrict__ cell,
+                                         const uint32_t *__restrict__ start, const DensityFields &f,
+                                         const NeighbourList &nl, const ParticleSoA &out,
+                                         uint32_t *__restrict__ key_next, const CellCount &cc, float *__restrict__ ax,
+                                         float *__restrict__ ay, float *__restrict__ az, const SceneTable &t,
+                                         const Scene &s, const Consts &k, uint32_t i, uint32_t *my, float4 *s_owner,
+                                         float4 *s_acc, uint16_t *s_items)
 {
-    static_assert(kGroupSlots % T == 0, "a workgroup must lie in one slot group");
     constexpr bool kLists = kMode == kNbLists;
-    constexpr int kLst = kMode != kNbMasks ? 0 : kQueue ? C + 2 : C;
-    __shared__ uint32_t lst[(kLst > kListCap ? kLst : kListCap) * T];
-    __shared__ float4 s_owner[kLists ? 2 * T : 1];
-    __shared__ float4 s_acc[kLists ? 2 * T : 1];
-    __shared__ uint16_t s_items[kLists ? kLevelWindow * T : 1];
-    const uint32_t first = xcd_block(blockIdx.x, gridDim.x) * (uint32_t) T, i = first + threadIdx.x;
-    const Scene s = block_scene(t, first);
     const uint32_t li = i - s.poff;
     if (i >= t.nslots) return;
     if (!kRef) count_dead(cc, i, s);
@@ -2197,7 +2261,7 @@ __global__ __launch_bounds__(T) void k_forces_fused(ParticleSoA p, const uint32_
     const float vxi = p.vx[i], vyi = p.vy[i], vzi = p.vz[i];
     float a0, a1, a2;
     if (kMode == kNbWalk) {
-        sph_accel<kRef, T, U>(p, cell, start, f, nl, lst + threadIdx.x, i, li, s, k, xi, yi, zi, vxi, vyi, vzi, a0, a1,
+        sph_accel<kRef, T, U>(p, cell, start, f, nl, my, i, li, s, k, xi, yi, zi, vxi, vyi, vzi, a0, a1,
                         a2);
     } else {
         const BufView bv = buf_view(p, f, s);
@@ -2214,14 +2278,14 @@ __global__ __launch_bounds__(T) void k_forces_fused(ParticleSoA p, const uint32_
         } else {
             overflow = cnt_i != 0;
             if (!overflow && kQueue)
-                a = mask_sums_queue<kRef, T, C / 2>(bv, cell, start, nl.masks, lst + threadIdx.x, i, li, s, k, xi, yi, zi,
+                a = mask_sums_queue<kRef, T, C / 2>(bv, cell, start, nl.masks, my, i, li, s, k, xi, yi, zi,
                                               vxi, vyi, vzi, ai);
             else if (!overflow)
-                a = mask_sums<kRef, T, C, kStall>(bv, cell, start, nl.masks, lst + threadIdx.x, i, li, s, k, xi, yi, zi,
+                a = mask_sums<kRef, T, C, kStall>(bv, cell, start, nl.masks, my, i, li, s, k, xi, yi, zi,
                                             vxi, vyi, vzi, ai);
         }
         if (overflow)
-            a = walk_sums<kRef, T, U>(bv, cell, start, lst + threadIdx.x, i, li, s, k, xi, yi, zi, vxi, vyi, vzi, ai);
+            a = walk_sums<kRef, T, U>(bv, cell, start, my, i, li, s, k, xi, yi, zi, vxi, vyi, vzi, ai);
         accel_from_sums(a, rhoi, s, k, a0, a1, a2);
     }
     wall_accel(xi, yi, zi, vxi, vyi, vzi, s, k, a0, a1, a2);
@@ -2237,6 +2301,28 @@ __global__ __launch_bounds__(T) void k_forces_fused(ParticleSoA p, const uint32_
     const uint32_t c = hash_key<kRef>(nx, ny, nz, s, k.h);
     key_next[i] = c;
     if (!kRef && cc.count) count_key(cc, i, c);
+}
+
+template <int T, int U, int C, int kStall, bool kQueue, int kMode, bool kStoreAcc, bool kRef>
+__global__ __launch_bounds__(T) void k_forces_fused(ParticleSoA p, const uint32_t *__restrict__ cell,
+                                                    const uint32_t *__restrict__ start, DensityFields f,
+                                                    NeighbourList nl, ParticleSoA out,
+                                                    uint32_t *__restrict__ key_next, CellCount cc,
+                                                    float *__restrict__ ax, float *__restrict__ ay,
+                                                    float *__restrict__ az, SceneTable t, Consts k)
+{
+    static_assert(kGroupSlots % T == 0, "a workgroup must lie in one slot group");
+    constexpr bool kLists = kMode == kNbLists;
+    constexpr int kLst = kMode != kNbMasks ? 0 : kQueue ? C + 2 : C;
+    __shared__ uint32_t lst[(kLst > kListCap ? kLst : kListCap) * T];
+    __shared__ float4 s_owner[kLists ? 2 * T : 1];
+    __shared__ float4 s_acc[kLists ? 2 * T : 1];
+    __shared__ uint16_t s_items[kLists ? kLevelWindow * T : 1];
+    const uint32_t first = xcd_block(blockIdx.x, gridDim.x) * (uint32_t) T;
+    const Scene s = block_scene(t, first);
+    fused_of<T, U, C, kStall, kQueue, kMode, kStoreAcc, kRef>(p, cell, start, f, nl, out, key_next, cc, ax, ay, az, t,
+                                                              s, k, first + threadIdx.x, lst + threadIdx.x, s_owner,
+                                                              s_acc, s_items);
 }
 
 // ---------------------------------------------------------------- neighbour passes of small launches
@@ -2275,16 +2361,27 @@ __global__ __launch_bounds__(64) void k_density_split(ParticleSoA p, const uint3
     __shared__ float s_r2[kSplitList * 64];
     __shared__ uint16_t s_j[kSplitList * 64];
     __shared__ uint32_t s_state[64];   // accepted candidates in a lane's list, and (bit 31) whether its rows are done
+    static_assert(density_list_cap<8>() <= kSplitList, "the one-lane pass uses the same LDS");
     const uint32_t lane = threadIdx.x, sub = lane & 15u, g = lane >> 4;
     const uint32_t first = xcd_block(blockIdx.x, gridDim.x) * 16u, i = first + sub;
     const Scene s = block_scene(t, first);
-    if (first - s.poff >= s.n) return;
     const uint32_t li = i - s.poff;
     const bool live = li < s.n;
     const BufView bv = buf_view(p, f, s);
     const float xi = ldf(bv.px, li * 4u), yi = ldf(bv.py, li * 4u), zi = ldf(bv.pz, li * 4u);
+    const uint32_t key = live ? cell[i] : 0u;
+    if (is_crowded(crowd_word(nl.crowd, t.nslots))) {
+        const uint32_t blocks = (t.nslots + 63u) / 64u;
+        if (blockIdx.x >= blocks) return;
+        const uint32_t first1 = xcd_block(blockIdx.x, blocks) * 64u, i1 = first1 + lane;
+        const Scene s1 = block_scene(t, first1);
+        if (i1 < t.nslots && i1 - s1.poff < s1.n)
+            density_of<64, 8, false, true, kDiag, kRef>(p, cell, start, f, nl, nl.masks, s1, k, i1, s_r2 + lane);
+        return;
+    }
+    if (first - s.poff >= s.n) return;
     int x = 0, y = 0, z = 0;
-    if (live) cell_xyz<kRef>(cell[i], s, x, y, z);
+    if (live) cell_xyz<kRef>(key, s, x, y, z);
     const RowBounds rb = row_bounds(s, k, x, y, z, xi, yi, zi);
     int r = (int) (2u * g);
     const int rlast = g == 3u ? 8 : r + 1;
@@ -2391,10 +2488,26 @@ __global__ __launch_bounds__(64) void k_forces_split(ParticleSoA p, const uint32
                                                      float *__restrict__ ax, float *__restrict__ ay,
                                                      float *__restrict__ az, SceneTable t, Consts k)
 {
-    __shared__ uint32_t lst[kListCap * 64];
+    constexpr int kQueueWords = 48;   // as variant 12
+    static_assert(kQueueWords == 2 * kPhaseWords && kQueueWords >= kListCap, "one array for all paths");
+    __shared__ uint32_t lst[(kQueueWords + 2) * 64];
+    const uint32_t crowd = crowd_word(nl.crowd, t.nslots);
     const uint32_t lane = threadIdx.x, q = lane & 3u;
     const uint32_t first = xcd_block(blockIdx.x, gridDim.x) * 16u, i = first + (lane >> 2);
     const Scene s = block_scene(t, first);
+    if (is_crowded(crowd)) {
+        const uint32_t blocks = (t.nslots + 63u) / 64u;
+        if (blockIdx.x >= blocks) return;
+        const uint32_t first1 = xcd_block(blockIdx.x, blocks) * 64u, i1 = first1 + lane;
+        const Scene s1 = block_scene(t, first1);
+        if constexpr (kFused)
+            fused_of<64, 8, kQueueWords, 0, true, kNbMasks, kStoreAcc, kRef>(p, cell, start, f, nl, out, key_next, cc, ax,
+                                                                             ay, az, t, s1, k, i1, lst + lane, nullptr,
+                                                                             nullptr, nullptr);
+        else
+            phase_of<kRef, true>(p, cell, start, f, nl, ax, ay, az, t, s1, k, i1, lst + lane);
+        return;
+    }
     const uint32_t li = i - s.poff;
     if (i >= t.nslots) return;
     if (kFused && !kRef && q == 0u) count_dead(cc, i, s);
@@ -2694,11 +2807,11 @@ void launch_ref_place(const RefBuffers &r, const uint32_t *skey, const uint32_t 
 }
 
 void launch_ref_final(const RefBuffers &r, const uint32_t *gnew, const uint32_t *start, uint32_t *skey, uint32_t *perm,
-                      uint32_t *ocell, const SceneTable &t, hipStream_t st)
+                      uint32_t *ocell, uint32_t *crowd, const SceneTable &t, hipStream_t st)
 {
     if (t.nslots == 0) return;
     hipLaunchKernelGGL(k_ref_final, dim3(blocks_for(t.nslots, 256)), dim3(256), 0, st, gnew, (const uint32_t *) r.rk,
-                       start, skey, perm, ocell, t);
+                       start, skey, perm, ocell, crowd, t);
 }
 
 void launch_cell_table(const CellCount &cc, unsigned long long *state, uint32_t *start, uint32_t ncells, hipStream_t st,
@@ -2717,16 +2830,23 @@ void launch_place(const uint32_t *key, const CellCount &cc, unsigned long long *
 }
 
 void launch_gather(const ParticleSoA &src, const ParticleSoA &dst, const uint32_t *list, const uint32_t *skey,
-                   const uint32_t *start, uint32_t *perm, const SceneTable &t, hipStream_t st)
+                   const uint32_t *start, uint32_t *perm, uint32_t *crowd, const SceneTable &t, hipStream_t st)
 {
     if (t.nslots == 0) return;
-    hipLaunchKernelGGL(k_gather, dim3(blocks_for(t.nslots, 256)), dim3(256), 0, st, src, dst, list, skey, start, perm, t);
+    hipLaunchKernelGGL(k_gather, dim3(blocks_for(t.nslots, 256)), dim3(256), 0, st, src, dst, list, skey, start, perm,
+                       crowd, t);
 }
 
 void launch_cell_start(const uint32_t *sorted_keys, uint32_t n, uint32_t ncells, uint32_t *start, hipStream_t st)
 {
     hipLaunchKernelGGL(k_cell_start, dim3(blocks_for(n + 1, 256)), dim3(256), 0, st, sorted_keys, n, ncells,
                        start);
+}
+
+void launch_crowding(const uint32_t *skey, const uint32_t *start, uint32_t *crowd, const SceneTable &t, hipStream_t st)
+{
+    if (t.nslots == 0) return;
+    hipLaunchKernelGGL(k_crowding, dim3(blocks_for(t.nslots, 256)), dim3(256), 0, st, skey, start, crowd, t);
 }
 
 void launch_reorder(const ParticleSoA &src, const ParticleSoA &dst, const uint32_t *perm, uint32_t n,

@@ -179,6 +179,9 @@ sph_status step_noalloc(const sph_params *prm, const sph_device_state *st, uint3
     nl.kmax = 0;
     nl.mode = split_neighbours(n, n) ? kNbSplit : kNbMasks;
     nl.masks = u32(kOffMasks);
+    nl.crowd = u32(kOffRho) + kMaxN - kCrowdWords;   // no slot of a launch that has them
+    static_assert(kMaxN >= kSplitSlots + kCrowdWords, "the crowding lies behind the densities");
+    uint32_t *crowd = nl.mode == kNbSplit ? nl.crowd : nullptr;
     SceneTable tab{scene_d, nullptr, n};
     const Consts k = make_consts();
 
@@ -191,7 +194,7 @@ sph_status step_noalloc(const sph_params *prm, const sph_device_state *st, uint3
         // grid phase (as run_grid)
         launch_cell_table(counts, state, cstart, tabled, stream);
         launch_place(key_h, counts, state, cstart, tabled, list, key_s, tab, stream);
-        launch_gather(soa(cur, idc), soa(1 - cur, 1 - idc), list, key_s, cstart, perm, tab, stream);
+        launch_gather(soa(cur, idc), soa(1 - cur, 1 - idc), list, key_s, cstart, perm, crowd, tab, stream);
         cur = 1 - cur;
         idc = 1 - idc;
         // density, then forces + walls + integrate + the next step's keys

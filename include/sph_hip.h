@@ -319,7 +319,8 @@ sph_status sph_set_graphs(sph_ctx *ctx, int enable);
  *                        was created with max_neighbours > 0);
  *   SPH_NEIGHBOURS_MASKS reads per-row masks of the accepted candidates the density pass
  *                        kept (576 bytes per slot); up to 40,960 slots in use, 16-bit
- *                        neighbour slots kept there, four lanes to a particle.
+ *                        neighbour slots kept there, four lanes to a particle (unless
+ *                        the particles lie too close together for that to be faster).
  * A new context uses variant 12 and SPH_NEIGHBOURS_MASKS, or SPH_NEIGHBOURS_LISTS when it
  * was created with max_neighbours > 0. Results are identical for every choice. */
 #define SPH_NUM_VARIANTS 21
