@@ -139,3 +139,29 @@ def test_a_crowded_cell_does_not_hold_up_the_sort(hip):
             ms.append(min(t[1:]))
     print("spread %.3f ms, crowded %.3f ms" % tuple(ms), flush=True)
     assert ms[1] < 6.0 * ms[0]
+
+
+@pytest.mark.parametrize("res,n,more", [(30, 200_000, 220), (102, 200_000, 220), (102, 1_200_000, 260),
+                                        (257, 200_000, 0), (385, 8_000_000, 0)])
+def test_digit_sort_across_key_widths(hip, res, n, more):
+    """The stable sort by digits: two 8-bit passes (30^3 cells), three (102^3) and three of 10
+    bits (257^3, 385^3; with 8,000,000 particles the histograms fill 489 scan tiles). An
+    empty scene of more^3 cells beside the first makes the cells too many to count."""
+    lib = hip._lib
+    h = float(hip.scenes.H)
+    boxes = [float(np.float32((r - 0.5) * h)) for r in (res, more) if r]
+    assert sum(r ** 3 for r in (res, more)) > (8 << 20) + 6 * n
+    rng = np.random.default_rng([res, n])
+    pos = ((rng.random((n, 3)) - 0.5) * boxes[0]).astype(np.float32)
+    print("%d^3 cells, %d particles" % (res, n), flush=True)
+    with hip.SceneBatch([(boxes[0], n)] + [(b, 256) for b in boxes[1:]]) as b:
+        b.upload(0, pos)
+        assert b.grid(0)[0] == (res, res, res)
+        b.phase(lib.PHASE_GRID)
+        pre = b.debug(0, lib.DEBUG_CELL_PRESORT)
+        want = np.argsort(pre, kind="stable").astype(np.uint32)
+        np.testing.assert_array_equal(b.debug(0, lib.DEBUG_PERM), want)
+        np.testing.assert_array_equal(b.debug(0, lib.DEBUG_CELL), pre[want])
+        np.testing.assert_array_equal(b.debug(0, lib.DEBUG_CELL_START),
+                                      np.searchsorted(pre[want], np.arange(res ** 3 + 1), side="left").astype(np.uint32))
+        np.testing.assert_array_equal(b.download(0, by_id=False)[2], want)

@@ -47,3 +47,57 @@ def test_full_rows(hip, orc, sizes):
             p, w, _ = b.download(0)
         assert_bits_equal(p, want["pos"], "variant %d positions" % v)
         assert_bits_equal(w, want["vel"], "variant %d velocities" % v)
+
+
+def lattice_block(h, side, spacing, rng):
+    """side^3 sites `spacing` apart, jittered by 0.01 h, from the corner of a 0.4 m box."""
+    g = np.arange(side) * spacing - 0.15
+    pos = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3)
+    return (pos + rng.uniform(-0.01 * h, 0.01 * h, pos.shape)).astype(np.float32)
+
+
+@pytest.mark.parametrize("reference", [False, True])
+@pytest.mark.parametrize("scene,steps", [("loose", 8), ("six words a row", 3), ("twelve words a row", 2),
+                                         ("rows too long", 2)])
+def test_variants_on_the_masks(hip, orc, scene, steps, reference):
+    """Every variant where the queues drain once, several times and not at all (rows of more
+    than 512 candidates are walked); the phases and the accelerations with the default one.
+    The reference order is compiled in one shape."""
+    lib = hip._lib
+    h = float(hip.scenes.H)
+    rng = np.random.default_rng(31)
+    if scene == "loose":
+        pos = hip.scenes.lattice(15, 16, 17, 0.4, jitter_h=0.01, seed=3)
+    elif scene == "rows too long":
+        pos = (rng.random((3000, 3)) * 0.09 - 0.2).astype(np.float32)
+    else:
+        pos = lattice_block(h, 16 if scene == "six words a row" else 15, h / (4 if scene == "six words a row" else 5), rng)
+    vel = rng.normal(0, 0.3, pos.shape).astype(np.float32)
+    flags = lib.FLAG_REFERENCE_ORDER if reference else 0
+    o = orc.OracleSim(0.4, len(pos))
+    o.add_particles(pos, vel)
+    o.set_order_mode(orc.ORDER_REFERENCE if reference else orc.ORDER_CANONICAL)
+    o.step(steps)
+    want = o.state()
+    assert np.isfinite(want["vel"]).all()
+    for v in [12] if reference else range(lib.NUM_VARIANTS):
+        print("%s, reference order %s, variant %d" % (scene, reference, v), flush=True)
+        with hip.HIPGridParticleSimulator(0.4, capacity=CAPACITY, flags=flags) as sim:
+            sim.upload(pos, vel)
+            lib.check(sim._lib.sph_set_variant(sim._ctx, v, lib.NEIGHBOURS_MASKS))
+            sim.advance(steps)
+            p, w, _ = sim.download()
+        assert_bits_equal(p, want["pos"], "variant %d positions" % v)
+        assert_bits_equal(w, want["vel"], "variant %d velocities" % v)
+    for fused in (True, False):
+        with hip.HIPGridParticleSimulator(0.4, capacity=CAPACITY, flags=flags | lib.FLAG_DIAGNOSTICS, fused=fused) as sim:
+            sim.upload(pos, vel)
+            for _ in range(steps):
+                sim.step()
+            p, w, _ = sim.download()
+            ids = sim.debug(lib.DEBUG_IDS)
+            assert_bits_equal(sim.debug(lib.DEBUG_DENSITY), want["density"][ids], "density, fused %s" % fused)
+            if fused:   # the phases' acceleration is the forces' alone until the walls' are added
+                assert_bits_equal(sim.debug(lib.DEBUG_ACCEL), want["acc"][ids], "acceleration")
+        assert_bits_equal(p, want["pos"], "positions, fused %s" % fused)
+        assert_bits_equal(w, want["vel"], "velocities, fused %s" % fused)
