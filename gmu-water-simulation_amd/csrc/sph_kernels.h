@@ -251,13 +251,16 @@ void launch_crowding(const uint32_t *skey, const uint32_t *start, uint32_t *crow
 void launch_reorder(const ParticleSoA &src, const ParticleSoA &dst, const uint32_t *perm, uint32_t n,
                     hipStream_t st);
 
-// pos[3*id + c] (and vel) for slots first .. first+n-1; ids outside 0..n-1 set *bad.
+// n particles from xyz triples, at rest without vel, with ids id_base .. without ids, into
+// slots first .. first+n-1 (ocell, if given, 0). The host arrays are pinned.
 void launch_unpack(const float *pos, const float *vel, const uint32_t *ids, uint32_t id_base, const ParticleSoA &p,
                    uint32_t *ocell, uint32_t first, uint32_t n, hipStream_t st);
+// pos[3*id + c] (and vel) of slots first .. first+n-1, by way of at[id] = slot; ids outside
+// 0..n-1 set *bad.
 void launch_pack_by_id(const ParticleSoA &p, uint32_t first, uint32_t n, uint32_t *at, float *pos, float *vel,
                        uint32_t *bad, hipStream_t st);
 
-// Density pass: density, p/rho^2, 1/rho and the neighbour lists. `ref`: the
+// Density pass: density, the force pass's records and the neighbours. `ref`: the
 // scenes use the reference order (kOrderReference; one kernel shape).
 void launch_density(const ParticleSoA &p, const uint32_t *cell, const uint32_t *start, const DensityFields &f,
                     const NeighbourList &nl, const SceneTable &t, const Consts &k, int variant, bool ref,

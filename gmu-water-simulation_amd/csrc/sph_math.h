@@ -210,7 +210,7 @@ __device__ __forceinline__ void div3_small_divisor(float a0, float a1, float a2,
     }
 }
 
-// a_c / b with rb = 1/b rounded to double: zero or subnormal results of a
+// a_c / b with rb = 1/b to within 2^-52: zero or subnormal results of a
 // non-zero a take the IEEE division (b is re-read through `divisor` only then).
 template <typename Divisor>
 __device__ __forceinline__ void div3_rcp(float a0, float a1, float a2, double rb, Divisor divisor, float &q0,
